@@ -147,6 +147,11 @@ void launch_vl_stage(hipStream_t st, const BoxDesc* boxes, const TilePlan& plan,
 // workgroups of a fused stage resident per CU (occupancy of the kernel as compiled)
 template <class real, int RS>
 int vl_stage_blocks_per_cu(int kind, int shape);
+// kind 3 in FP64: k_vl_char, each cell's edge values formed once (tile shapes 0 and 1)
+template <int RS>
+void launch_vl_char(hipStream_t st, const BoxDesc* boxes, const TilePlan& plan, const StageArgs<double>& a, int shape);
+template <int RS>
+int vl_char_blocks_per_cu(int shape);
 constexpr int vs_kind(bool corrector, int recon) { return corrector ? 1 + recon : 0; }
 
 }  // namespace imhd

@@ -858,7 +858,7 @@ __global__ __launch_bounds__(TX * TY, VS_WAVES) void k_vl_stage(const BoxDesc* _
 }
 
 // kind: 0 predictor, 1 PLM corrector, 2 PPM-primitive corrector, 3 PPM-characteristic
-// corrector; shape 2 exists in FP32 only
+// corrector (FP32; FP64 runs k_vl_char); shape 2 exists in FP32 only
 template <class real, int RS, int KIND>
 void launch_vl_stage_k(hipStream_t st, const BoxDesc* boxes, const TilePlan& plan, const StageArgs<real>& a,
                        int shape) {
@@ -907,7 +907,9 @@ int vl_stage_blocks_per_cu(int kind, int shape) {
         case 5:
             if constexpr (sizeof(real) == 4) return vl_stage_blocks_per_cu_k<real, RS, 5>(shape);
             return vl_stage_blocks_per_cu_k<real, RS, 0>(shape);
-        default: return vl_stage_blocks_per_cu_k<real, RS, 3>(shape);
+        default:
+            if constexpr (sizeof(real) == 4) return vl_stage_blocks_per_cu_k<real, RS, 3>(shape);
+            return vl_char_blocks_per_cu<RS>(shape);
     }
 }
 
@@ -927,7 +929,10 @@ void launch_vl_stage(hipStream_t st, const BoxDesc* boxes, const TilePlan& plan,
             if constexpr (sizeof(real) == 4) launch_vl_stage_k<real, RS, 5>(st, boxes, plan, a, shape);
             else launch_vl_stage_k<real, RS, 0>(st, boxes, plan, a, shape);
             break;
-        default: launch_vl_stage_k<real, RS, 3>(st, boxes, plan, a, shape); break;
+        default:   // FP64 shares each cell's edge values between its faces
+            if constexpr (sizeof(real) == 4) launch_vl_stage_k<real, RS, 3>(st, boxes, plan, a, shape);
+            else launch_vl_char<RS>(st, boxes, plan, a, shape);
+            break;
     }
 }
 
