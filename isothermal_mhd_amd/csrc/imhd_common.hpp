@@ -62,6 +62,16 @@ __device__ __forceinline__ unsigned xcd_block(unsigned w, unsigned G) {
     return base + idx;
 }
 
+// How many cells of [lo, n + hi] along every axis are periodic images of cell (i, j, k), 0
+// if it is itself a ghost cell: the density floor's count over the reference's update range,
+// for a step that updates fewer ghost cells (boxes of at least nb cells per axis).
+__device__ __forceinline__ unsigned floor_images(int n0, int n1, int n2, int i, int j, int k, int lo, int hi) {
+    auto along = [&](int v, int n) {
+        return v < 1 || v > n ? 0u : 1u + (v - n >= lo ? 1u : 0u) + (v <= hi ? 1u : 0u);
+    };
+    return along(i, n0) * along(j, n1) * along(k, n2);
+}
+
 // Maps this thread to (box, i, j, k).  Returns false for padding threads.
 __device__ __forceinline__ bool plan_item(const Plan& p, int& box, int& i, int& j, int& k) {
     unsigned blk = xcd_block(blockIdx.x, gridDim.x);

@@ -125,6 +125,7 @@ struct StageArgs {
     int ccb_lo_shift;
     real* comp[4];          // Kahan terms (final stage of the FP32 path) or null
     unsigned int* floor_count;
+    int img, img_lo, img_hi;    // img: a floored cell counts for its images in [img_lo, n + img_hi]
     unsigned long long* cmax;   // non-null: CFL speed of the new interior cells
     unsigned long long* smax;
     double cs;

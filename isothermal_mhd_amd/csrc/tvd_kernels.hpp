@@ -53,6 +53,7 @@ struct TvdHalfArgs {
     real* dst[7];          // half state (the slot of the sweep's normal field is not written)
     const double* dt;
     unsigned int* floor_count;
+    int img, img_lo, img_hi;   // img: a floored cell counts for its images in [img_lo, n + img_hi]
     int dir;
 };
 

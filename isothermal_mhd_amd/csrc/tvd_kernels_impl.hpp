@@ -710,7 +710,7 @@ __global__ __launch_bounds__(256) void k_tvd_half3(const BoxDesc* __restrict__ b
 #pragma unroll
     for (int d = 0; d < 3; d++) tvd_half_calc(a, d, c, st, q, dB, dtd, hq[d], bt[d], fl[d]);
     const unsigned nf = (unsigned)fl[0] + (unsigned)fl[1] + (unsigned)fl[2];
-    if (nf) atomicAdd(a.floor_count, nf);
+    if (nf) atomicAdd(a.floor_count, a.img ? nf * floor_images(B.n[0], B.n[1], B.n[2], i, j, k, a.img_lo, a.img_hi) : nf);
 #pragma unroll
     for (int d = 0; d < 3; d++) {
 #pragma unroll

@@ -550,7 +550,7 @@ __global__ __launch_bounds__(TX * TY, 2) void k_vl_char(const BoxDesc* __restric
                 double v = q0v - dtdx * div[f];
                 if (f == 0 && v < MIN_DENS) {
                     v = MIN_DENS;
-                    atomicAdd(a.floor_count, 1u);
+                    atomicAdd(a.floor_count, a.img ? floor_images(n0, n1, n2, i, j, k, a.img_lo, a.img_hi) : 1u);
                 }
                 a.dst.q[f][c] = v;
                 nq[f] = v;

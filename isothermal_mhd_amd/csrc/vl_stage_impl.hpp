@@ -772,7 +772,7 @@ __global__ __launch_bounds__(TX * TY, VS_WAVES) void k_vl_stage(const BoxDesc* _
                 if (f == 0 && v < (real)MIN_DENS) {
                     v = (real)MIN_DENS;
                     if (!PRED && a.comp[0] != nullptr) a.comp[0][c] = real(0);
-                    atomicAdd(a.floor_count, 1u);
+                    atomicAdd(a.floor_count, a.img ? floor_images(n0, n1, n2, i, j, k, a.img_lo, a.img_hi) : 1u);
                 }
                 a.dst.q[f][c] = v;
                 nq[f] = v;
