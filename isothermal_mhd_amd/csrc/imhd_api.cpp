@@ -159,6 +159,7 @@ struct imhd_ctx {
     int vseg = 16;       // z-segment length of the fused stages when vrounds = 0
     int vrounds = 4;     // > 0: fused-stage workgroups = vrounds x resident workgroups of the GPU
     int ncu = 0;         // compute units of the device
+    int sweep_waves = 0; // resident waves of the y/z Roe-TVD sweep on the device
     int vshape = 0;      // tile shape of the fused stages (0: 16 x 16, 1: 32 x 16; FP32 default 1)
     int vshape_c = 0;    // tile shape of the fused corrector (the autotuner may choose it apart)
     bool vsh = true;     // FP32 PLM corrector from LDS-held primitives with shared slopes (kind 4)
@@ -219,6 +220,24 @@ int put_plan(imhd_ctx* c, T*& d, const std::vector<T>& h) {
     HIPCK(c, hipStreamSynchronize(c->st));   // launches that read the old entry
     HIPCK(c, hipMemcpy(d, h.data(), bytes, hipMemcpyHostToDevice));
     return 0;
+}
+
+// Faces a thread of the y and z Roe-TVD sweeps marches.  A segment costs two faces more
+// than it writes, and a launch as many rounds of the resident waves as it fills: the length
+// with the least rounds x (length + 2), the longest of those.  64^3 (4900 columns) then has
+// three faces per segment and one round of waves instead of a third of one with eight.
+// (The boxes of an ensemble share a launch and are cut alike: 32 faces, 8 in small boxes.)
+int sweep_segment(const imhd_ctx* c, long long columns, int faces) {
+    if (c->nbox > 1) return faces >= 128 ? 32 : 8;
+    const long long slots = std::max(1, c->sweep_waves);
+    int best = 32;
+    long long cost = -1;
+    for (int s = 32; s >= 2; s--) {
+        const long long waves = (columns * ((faces + s - 1) / s) + 63) / 64;
+        const long long v = (waves + slots - 1) / slots * (s + 2);
+        if (cost < 0 || v < cost) cost = v, best = s;
+    }
+    return best;
 }
 
 // Trimmed native steps.  The reference's stages update as many ghost cells as their inputs
@@ -340,15 +359,15 @@ int build_plan(imhd_ctx* c, PlanDev& p, int which, int dir, int seg = 0, bool tr
         pb.start = run;
         long long cnt = (long long)pb.r[0] * pb.r[1] * pb.r[2];
         if (which == 27 || which == 28) {
-            // fused Roe-TVD sweep: x -- one wave per (row, TVD_XSEG faces);
-            // y, z -- one thread per (x, transverse, segment of seg faces along the sweep)
+            // fused Roe-TVD sweep: x -- waves of TVD_XSEG + 2 entries of the flat list of
+            // all rows, each row's faces with the one before and the one after; y, z -- one
+            // thread per (x, transverse, segment of seg faces along the sweep)
             if (dir == 0) {
-                pb.seg = TVD_XSEG;
-                pb.zn = (pb.r[0] + TVD_XSEG - 1) / TVD_XSEG;
-                cnt = (long long)pb.r[1] * pb.r[2] * pb.zn * 64;
+                const long long entries = (long long)pb.r[1] * pb.r[2] * (pb.r[0] + 2);
+                cnt = (entries - 2 + TVD_XSEG - 1) / TVD_XSEG * 64;
             } else {
                 const int ta = dir == 1 ? 2 : 1;
-                pb.seg = pb.r[dir] >= 128 ? 32 : 8;
+                pb.seg = sweep_segment(c, (long long)pb.r[0] * pb.r[ta], pb.r[dir]);
                 pb.zn = (pb.r[dir] + pb.seg - 1) / pb.seg;
                 cnt = (long long)pb.r[0] * pb.r[ta] * pb.zn;
             }
@@ -2267,6 +2286,8 @@ int imhd_create_ensemble(const imhd_config* cfg, int nbox, imhd_ctx** out) {
     HIPCK(c, hipMemcpy(c->cour, v.data(), 8 * nbox, hipMemcpyHostToDevice));
     std::fill(v.begin(), v.end(), 1.0e-15);  // driver.f90:249
     HIPCK(c, hipMemcpy(c->dt, v.data(), 8 * nbox, hipMemcpyHostToDevice));
+    if (g.integrator == IMHD_TVD)
+        c->sweep_waves = c->ncu * (g.precision == 64 ? tvd_sweep_waves_per_cu<double>() : tvd_sweep_waves_per_cu<float>());
     c->plans_h.resize(PLAN_SLOTS * plan_slot(nbox));
     HIPCK(c, hipMalloc(&c->plans, c->plans_h.size()));
     for (int d = 0; d < 3; d++) {

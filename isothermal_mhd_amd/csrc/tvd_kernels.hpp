@@ -5,7 +5,7 @@
 
 namespace imhd {
 
-// flux faces per wave of the fused x sweep (64 lanes: 62 faces + one neighbour face on
+// entries a wave of the fused x sweep advances by (64 lanes: 62 faces + one neighbour on
 // each side)
 constexpr int TVD_XSEG = 62;
 
@@ -92,6 +92,9 @@ void launch_tvd_flux(const Launch& L, const TvdSweepArgs<real>& a);
 // Fused eigen-system + flux sweep (plans: build_plan case 27 for x, 28 for y / z)
 template <class real>
 void launch_tvd_sweep(const Launch& L, const TvdSweepArgs<real>& a);
+// resident waves of the y / z sweep per CU (occupancy of the kernel as compiled)
+template <class real>
+int tvd_sweep_waves_per_cu();
 template <class real>
 void launch_tvd_hlle(const Launch& L, const TvdSweepArgs<real>& a);
 template <class real>

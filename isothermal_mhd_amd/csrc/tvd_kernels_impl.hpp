@@ -319,10 +319,13 @@ __global__ __launch_bounds__(256) void k_tvd_flux(const BoxDesc* __restrict__ bo
 // the chip).  The sweep's flux faces [lo, lo + r) per axis come from a face plan (build_plan
 // cases 17 / 19); each face's flux needs g~_k of its two neighbours along the sweep.
 //
-// x sweep: one wave per (row, segment of TVD_XSEG = 62 flux faces).  Lane l forms g~_k
-// and alpha_k of face x0 - 1 + l; lanes 1 .. 62 then take their neighbours' g~_k by wave
-// shuffles and form the flux of their own face from the states they already hold.  No
-// LDS and no barrier; every lane of the wave reaches the shuffles.
+// x sweep: the rows' faces, each row with the face before its first and after its last, form
+// one flat list; a wave takes TVD_XSEG + 2 = 64 of its entries and the next wave begins
+// TVD_XSEG further.  Lane l forms g~_k and alpha_k of its entry; lanes 1 .. 62 then take
+// their neighbours' g~_k (of the same row, by the two extra entries) by wave shuffles and
+// form the flux of their own face from the states they already hold.  No LDS and no
+// barrier; every lane of the wave reaches the shuffles.  Rows cut into segments of 62 faces
+// each left most of a row's last wave idle: at 200^3 (205 faces) a fifth of the lanes.
 template <class real>
 __global__ __launch_bounds__(256) void k_tvd_sweep_x(const BoxDesc* __restrict__ boxes, Plan plan, TvdSweepArgs<real> a) {
     const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
@@ -339,22 +342,25 @@ __global__ __launch_bounds__(256) void k_tvd_sweep_x(const BoxDesc* __restrict__
         b = lo;
     }
     const PlanBox& pb = plan.boxes[b];
-    const long long wseg = (gw - pb.start) >> 6;   // (row, segment) of this wave
-    const int nseg = pb.zn;
-    if (wseg >= (long long)pb.r[1] * pb.r[2] * nseg) return;   // whole wave
+    const unsigned len = (unsigned)pb.r[0] + 2u, rows = (unsigned)pb.r[1] * (unsigned)pb.r[2];
+    const unsigned wv = __builtin_amdgcn_readfirstlane((unsigned)((gw - pb.start) >> 6));
+    const unsigned long long e0 = (unsigned long long)wv * TVD_XSEG;   // this wave's first entry
+    if (e0 + 2 >= (unsigned long long)rows * len) return;              // whole wave
     const int lane = (int)(threadIdx.x & 63);
-    const int sgi = (int)(wseg % nseg);
-    const long long row = wseg / nseg;
-    const int j = pb.lo[1] + (int)(row % pb.r[1]);
-    const int k = pb.lo[2] + (int)(row / pb.r[1]);
-    const int x0 = pb.lo[0] + sgi * TVD_XSEG;
-    const int x1 = min(x0 + TVD_XSEG - 1, pb.lo[0] + pb.r[0] - 1);   // last flux face of the segment
-    const int x = x0 - 1 + lane;                                     // this lane's face
-    const bool eig = x <= x1 + 1;
+    const unsigned row0 = (unsigned)(e0 / len), off = (unsigned)(e0 - (unsigned long long)row0 * len) + (unsigned)lane;
+    const unsigned up = len >= 64u ? (off >= len ? 1u : 0u) : off / len;   // rows after row0
+    const int x = pb.lo[0] - 1 + (int)(off - up * len);       // this lane's face
+    const bool eig = row0 + up < rows;
+    unsigned jr = row0 % (unsigned)pb.r[1] + (eig ? up : 0u), kr = row0 / (unsigned)pb.r[1];
+    while (jr >= (unsigned)pb.r[1]) {
+        jr -= (unsigned)pb.r[1];
+        kr++;
+    }
+    const int j = pb.lo[1] + (int)jr, k = pb.lo[2] + (int)kr;
     const BoxDesc& B = boxes[b];
     real uL[7], uR[7], ck[6], gt[6], dtdx, dxdt;
     tvd_dts(a, B, b, dtdx, dxdt);
-    const long long c = cell_index(B, eig ? x : x0, j, k);
+    const long long c = cell_index(B, eig ? x : pb.lo[0], j, k);
     if (eig) {
         tvd_load(a, c, uL);
         tvd_load(a, c + 1, uR);
@@ -369,7 +375,7 @@ __global__ __launch_bounds__(256) void k_tvd_sweep_x(const BoxDesc* __restrict__
         gm[w] = __shfl_up(gt[w], 1, 64);
         gp[w] = __shfl_down(gt[w], 1, 64);
     }
-    if (lane >= 1 && lane <= TVD_XSEG && x <= x1) {
+    if (lane >= 1 && lane <= TVD_XSEG && eig && x >= pb.lo[0] && x < pb.lo[0] + pb.r[0]) {
         real F[7];
         tvd_flux_face(uL, uR, (real)a.cs, dtdx, dxdt, gm, gt, gp, ck, F);
         tvd_store(a, c, F);
@@ -906,6 +912,12 @@ void launch_tvd_sweep(const Launch& L, const TvdSweepArgs<real>& a) {
         hipLaunchKernelGGL((k_tvd_sweep_m<real>), dim3(L.blocks()), dim3(256), 0, L.stream, L.boxes, L.plan, a);
 }
 template <class real>
+int tvd_sweep_waves_per_cu() {
+    int n = 0;
+    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_tvd_sweep_m<real>, 256, 0);
+    return 4 * (e == hipSuccess && n > 0 ? n : 1);
+}
+template <class real>
 void launch_tvd_hlle(const Launch& L, const TvdSweepArgs<real>& a) {
     if (L.plan.total > 0) hipLaunchKernelGGL((k_tvd_hlle<real>), dim3(L.blocks()), dim3(256), 0, L.stream, L.boxes, L.plan, a);
 }
@@ -944,6 +956,7 @@ void launch_tvd_max_speed(const Launch& L, const QPtrs<real>& q, double cs, unsi
     template void launch_tvd_eig<T>(const Launch&, const TvdSweepArgs<T>&);         \
     template void launch_tvd_flux<T>(const Launch&, const TvdSweepArgs<T>&);        \
     template void launch_tvd_sweep<T>(const Launch&, const TvdSweepArgs<T>&);       \
+    template int tvd_sweep_waves_per_cu<T>();                                       \
     template void launch_tvd_hlle<T>(const Launch&, const TvdSweepArgs<T>&);        \
     template void launch_tvd_corner<T>(const Launch&, const TvdCornerArgs<T>&);     \
     template void launch_tvd_center<T>(const Launch&, const TvdCenterArgs<T>&);     \
