@@ -222,10 +222,10 @@ int put_plan(imhd_ctx* c, T*& d, const std::vector<T>& h) {
     return 0;
 }
 
-// Faces a thread of the y and z Roe-TVD sweeps marches.  A segment costs two faces more
+// Faces a thread of the FP32 y and z Roe-TVD sweeps marches.  A segment costs two faces more
 // than it writes, and a launch as many rounds of the resident waves as it fills: the length
-// with the least rounds x (length + 2), the longest of those.  64^3 (4900 columns) then has
-// three faces per segment and one round of waves instead of a third of one with eight.
+// with the least rounds x (length + 2), the longest of those (200^3: 3.32 -> 3.18 ms per
+// step with the flat x sweep).
 // (The boxes of an ensemble share a launch and are cut alike: 32 faces, 8 in small boxes.)
 int sweep_segment(const imhd_ctx* c, long long columns, int faces) {
     if (c->nbox > 1) return faces >= 128 ? 32 : 8;
@@ -359,14 +359,20 @@ int build_plan(imhd_ctx* c, PlanDev& p, int which, int dir, int seg = 0, bool tr
         pb.start = run;
         long long cnt = (long long)pb.r[0] * pb.r[1] * pb.r[2];
         if (which == 27 || which == 28) {
-            // fused Roe-TVD sweep: x -- waves of TVD_XSEG + 2 entries of the flat list of
-            // all rows, each row's faces with the one before and the one after; y, z -- one
-            // thread per (x, transverse, segment of seg faces along the sweep)
+            // fused Roe-TVD sweeps (tvd_kernels_impl.hpp).  x: waves of 64 entries of the flat
+            // list of all rows' faces (FP64: cells).  y, z: FP64 workgroups of TVD_X64 columns
+            // and TVD_ROWS64 entries of the flat list of their faces; FP32 one thread per (x,
+            // transverse, segment of seg faces along the sweep)
+            const bool f64 = c->prec == 64;
+            const int ta = dir == 1 ? 2 : 1;
             if (dir == 0) {
-                const long long entries = (long long)pb.r[1] * pb.r[2] * (pb.r[0] + 2);
-                cnt = (entries - 2 + TVD_XSEG - 1) / TVD_XSEG * 64;
+                const long long rows = (long long)pb.r[1] * pb.r[2];
+                cnt = f64 ? (rows * (pb.r[0] + 3) - 3 + TVD_XSEG64 - 1) / TVD_XSEG64 * 64
+                          : (rows * (pb.r[0] + 2) - 2 + TVD_XSEG - 1) / TVD_XSEG * 64;
+            } else if (f64) {
+                const long long cols = (long long)((pb.r[0] + TVD_X64 - 1) / TVD_X64) * pb.r[ta];
+                cnt = (cols * (pb.r[dir] + 2) - 2 + TVD_ROWS64 - 3) / (TVD_ROWS64 - 2) * 256;
             } else {
-                const int ta = dir == 1 ? 2 : 1;
                 pb.seg = sweep_segment(c, (long long)pb.r[0] * pb.r[ta], pb.r[dir]);
                 pb.zn = (pb.r[dir] + pb.seg - 1) / pb.seg;
                 cnt = (long long)pb.r[0] * pb.r[ta] * pb.zn;
@@ -2291,8 +2297,7 @@ int imhd_create_ensemble(const imhd_config* cfg, int nbox, imhd_ctx** out) {
     HIPCK(c, hipMemcpy(c->cour, v.data(), 8 * nbox, hipMemcpyHostToDevice));
     std::fill(v.begin(), v.end(), 1.0e-15);  // driver.f90:249
     HIPCK(c, hipMemcpy(c->dt, v.data(), 8 * nbox, hipMemcpyHostToDevice));
-    if (g.integrator == IMHD_TVD)
-        c->sweep_waves = c->ncu * (g.precision == 64 ? tvd_sweep_waves_per_cu<double>() : tvd_sweep_waves_per_cu<float>());
+    if (g.integrator == IMHD_TVD && g.precision == 32) c->sweep_waves = c->ncu * tvd_sweep_waves_per_cu();
     c->plans_h.resize(PLAN_SLOTS * plan_slot(nbox));
     HIPCK(c, hipMalloc(&c->plans, c->plans_h.size()));
     for (int d = 0; d < 3; d++) {

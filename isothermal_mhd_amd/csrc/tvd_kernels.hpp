@@ -8,6 +8,9 @@ namespace imhd {
 // entries a wave of the fused x sweep advances by (64 lanes: 62 faces + one neighbour on
 // each side)
 constexpr int TVD_XSEG = 62;
+// FP64 sweeps: cells a wave of the x sweep advances by; x-neighbours and list entries of a
+// workgroup of the y / z sweeps, of which it forms TVD_ROWS64 - 2 fluxes
+constexpr int TVD_XSEG64 = 61, TVD_X64 = 8, TVD_ROWS64 = 32;
 
 // Directional sweep over cell states rotated so that the sweep direction is "x":
 // w[r] = q[perm(d, r)], slot 4 unused (each cell's own upper face field comes from bn).
@@ -92,8 +95,7 @@ void launch_tvd_flux(const Launch& L, const TvdSweepArgs<real>& a);
 // Fused eigen-system + flux sweep (plans: build_plan case 27 for x, 28 for y / z)
 template <class real>
 void launch_tvd_sweep(const Launch& L, const TvdSweepArgs<real>& a);
-// resident waves of the y / z sweep per CU (occupancy of the kernel as compiled)
-template <class real>
+// resident waves of the FP32 y / z sweep per CU (occupancy of the kernel as compiled)
 int tvd_sweep_waves_per_cu();
 template <class real>
 void launch_tvd_hlle(const Launch& L, const TvdSweepArgs<real>& a);

@@ -5,4 +5,9 @@
 
 namespace imhd {
 IMHD_INST_TVD(float)
+int tvd_sweep_waves_per_cu() {
+    int n = 0;
+    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_tvd_sweep_m<float>, 256, 0);
+    return 4 * (e == hipSuccess && n > 0 ? n : 1);
+}
 }  // namespace imhd

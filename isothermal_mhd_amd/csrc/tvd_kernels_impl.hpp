@@ -183,6 +183,16 @@ __device__ __forceinline__ real tvd_Q(real chi, real e) {
     if (fabs(chi) < real(2) * e) return real(0.25) * fdiv(chi * chi, e) + e;
     return fabs(chi);
 }
+// FP64, e constant: the correctly rounded quotient chi^2 / e from the correctly rounded 1/e
+// (Markstein 1990: one product, its exact remainder, one correction) instead of the general
+// division's 11 instructions; select instead of a branch.  Where chi^2 / e is too small for
+// the remainder to be exact, the sum with e does not see it.
+__device__ __forceinline__ double tvd_Q64(double chi, double e) {
+    if (e == 0.0) return fabs(chi);   // known when compiled
+    const double x = chi * chi, r = 1.0 / e;
+    const double q = x * r, quo = fma(fma(-e, q, x), r, q);
+    return fabs(chi) < 2.0 * e ? 0.25 * quo + e : fabs(chi);
+}
 
 // minmod limiter of the TVD module (isotvd_mod.f90:2426-2429)
 template <class real>
@@ -235,7 +245,22 @@ __device__ __forceinline__ void tvd_eig_face(const real* uL, const real* uR, rea
         gt[w] = real(0.5) * (Qk - chi * chi) * ck[w];
     }
 }
+// the same, FP64, keeping the face's waves for its flux
+__device__ __forceinline__ void tvd_eig_wave(const double* uL, const double* uR, double cs, double dtdx,
+                                             TvdWave<double>& W, double* gt, double* ck) {
+    tvd_wave(uL, uR, cs, W);
+    tvd_ck(uL, uR, cs, W, ck);
+#pragma unroll
+    for (int w = 0; w < 6; w++) {
+        const double chi = dtdx * W.ev[w];
+        gt[w] = 0.5 * (tvd_Q64(chi, tvd_eps(w)) - chi * chi) * ck[w];
+    }
+}
 
+template <class real>
+__device__ __forceinline__ void tvd_flux_wave(const TvdWave<real>& W, const real* uL, const real* uR, real cs, real dtdx,
+                                              real dxdt, const real* gm, const real* g0, const real* gp, const real* ck,
+                                              real* F);
 // Roe-TVD flux of one face from its states, its alpha_k and the g~_k of the face below
 // (gm), itself (g0) and above (gp) (isotvd_mod.f90:2400-2466); F[4] = 0.
 template <class real>
@@ -243,6 +268,12 @@ __device__ __forceinline__ void tvd_flux_face(const real* uL, const real* uR, re
                                               const real* gm, const real* g0, const real* gp, const real* ck, real* F) {
     TvdWave<real> W;
     tvd_wave(uL, uR, cs, W);
+    tvd_flux_wave(W, uL, uR, cs, dtdx, dxdt, gm, g0, gp, ck, F);
+}
+template <class real>
+__device__ __forceinline__ void tvd_flux_wave(const TvdWave<real>& W, const real* uL, const real* uR, real cs, real dtdx,
+                                              real dxdt, const real* gm, const real* g0, const real* gp, const real* ck,
+                                              real* F) {
     real FT[6] = {real(0), real(0), real(0), real(0), real(0), real(0)};
 #pragma unroll
     for (int w = 0; w < 6; w++) {
@@ -250,7 +281,9 @@ __device__ __forceinline__ void tvd_flux_face(const real* uL, const real* uR, re
         const real gk0 = tvd_lim(gm[w], g0[w]), gk1 = tvd_lim(g0[w], gp[w]);
         real gam = (fabs(ckw) > (real)ZERO) ? fdiv(gk1 - gk0, ckw) : real(0);
         real chi = dtdx * W.ev[w] + gam;
-        real Qk = tvd_Q(chi, (real)tvd_eps(w));
+        real Qk;
+        if constexpr (sizeof(real) == 8) Qk = tvd_Q64(chi, tvd_eps(w));
+        else Qk = tvd_Q(chi, (real)tvd_eps(w));
         real betak = Qk * ckw - (gk0 + gk1);
         real r[6];
         tvd_rcol(w, cs, W, r);
@@ -385,10 +418,9 @@ __global__ __launch_bounds__(256) void k_tvd_sweep_x(const BoxDesc* __restrict__
 // y / z sweep: threads along x (coalesced), each marching a segment of pb.seg flux faces
 // along the sweep axis with a three-face window of g~_k in registers.  Items enumerate
 // (x, transverse index, segment), x fastest.
-// FP64: at most 256 registers, two waves per SIMD (the unbounded allocation took 268 and
-// left one: 1371 us per call at 256^3; bounded, 6 registers spill).
+// FP32 only; FP64 runs k_tvd_sweep_x64 and k_tvd_sweep_yz64 below.
 template <class real>
-__global__ __launch_bounds__(256, sizeof(real) == 8 ? 2 : 1) void k_tvd_sweep_m(const BoxDesc* __restrict__ boxes, Plan plan,
+__global__ __launch_bounds__(256, 1) void k_tvd_sweep_m(const BoxDesc* __restrict__ boxes, Plan plan,
                                                                               TvdSweepArgs<real> a) {
     const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
     const long long g = (long long)blk * blockDim.x + threadIdx.x;
@@ -454,6 +486,138 @@ __global__ __launch_bounds__(256, sizeof(real) == 8 ? 2 : 1) void k_tvd_sweep_m(
             uA[r] = uB[r];
             uB[r] = uC[r];
         }
+    }
+}
+
+// FP64 sweeps.  FP64 is bound by its arithmetic (square roots of 20 and divisions of 14
+// instruction slots each), and the kernels above form a face's waves twice, once for g~_k
+// and once for its flux.  Here a thread forms one face: its waves stay in registers while
+// g~_k goes to the neighbours' threads (156 registers, three waves per SIMD; the marching
+// kernel took 256, two).  Values as above, bit for bit.  Per face at 161 x 144 x 130 (64^3):
+// x 62 -> 47 ps (88 -> 74), y and z 66 -> 50 ps (113 -> 76); 2.40 -> 2.10 ms per step (0.304 ->
+// 0.250).
+//
+// x: the flat list of k_tvd_sweep_x, over cells: a lane loads one cell and takes the next
+// one, with its velocities' divisions saved, from lane + 1; 61 faces per wave.
+// y, z: 8 x-neighbours by 32 entries of the flat list of all columns (each column's faces
+// with one before and one after), g~_k through LDS; 30 faces per workgroup and x.  8 cells
+// of a row are half a cache line: the other half is another workgroup's, from L2, which the
+// arithmetic hides.
+
+__device__ __forceinline__ double tvd_lane_up(double x) {   // the value of lane l + 1
+    const long long v = __double_as_longlong(x);
+    const int lo = __builtin_amdgcn_mov_dpp((int)(unsigned)v, 0x130, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(v >> 32), 0x130, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
+}
+
+static __global__ __launch_bounds__(256, 2) void k_tvd_sweep_x64(const BoxDesc* __restrict__ boxes, Plan plan,
+                                                          TvdSweepArgs<double> a) {
+    const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
+    const long long g = (long long)blk * 256 + threadIdx.x;
+    const long long gw = g - (threadIdx.x & 63);   // first item of this wave
+    if (gw >= plan.total) return;                  // whole wave
+    int b = 0;
+    if (plan.nbox > 1) {
+        int lo = 0, hi = plan.nbox - 1;
+        while (lo < hi) {
+            int mid = (lo + hi + 1) >> 1;
+            if (plan.boxes[mid].start <= gw) lo = mid; else hi = mid - 1;
+        }
+        b = lo;
+    }
+    const PlanBox& pb = plan.boxes[b];
+    // cells of a row's list: those of its faces, one more face on either side
+    const unsigned len = (unsigned)pb.r[0] + 3u, rows = (unsigned)pb.r[1] * (unsigned)pb.r[2];
+    const unsigned wv = __builtin_amdgcn_readfirstlane((unsigned)((gw - pb.start) >> 6));
+    const unsigned long long e0 = (unsigned long long)wv * TVD_XSEG64;   // this wave's first cell
+    if (e0 + 3 >= (unsigned long long)rows * len) return;                // whole wave
+    const int lane = (int)(threadIdx.x & 63);
+    const unsigned row0 = (unsigned)(e0 / len), off = (unsigned)(e0 - (unsigned long long)row0 * len) + (unsigned)lane;
+    const unsigned up = len >= 64u ? (off >= len ? 1u : 0u) : off / len;
+    const int x = pb.lo[0] - 1 + (int)(off - up * len);   // this lane's cell, and the face above it
+    const bool in = row0 + up < rows;
+    unsigned jr = row0 % (unsigned)pb.r[1] + (in ? up : 0u), kr = row0 / (unsigned)pb.r[1];
+    while (jr >= (unsigned)pb.r[1]) {
+        jr -= (unsigned)pb.r[1];
+        kr++;
+    }
+    const BoxDesc& B = boxes[b];
+    double dtdx, dxdt;
+    tvd_dts(a, B, b, dtdx, dxdt);
+    const long long c = cell_index(B, in ? x : pb.lo[0], pb.lo[1] + (int)jr, pb.lo[2] + (int)kr);
+    double uL[7], uR[7], ck[6], gt[6], gm[6], gp[6];
+    tvd_load(a, c, uL);
+#pragma unroll
+    for (int r = 0; r < 7; r++) uR[r] = tvd_lane_up(uL[r]);   // lane 63 and a row's last cell: unused
+    TvdWave<double> W;
+    tvd_eig_wave(uL, uR, a.cs, dtdx, W, gt, ck);
+#pragma unroll
+    for (int w = 0; w < 6; w++) {
+        gm[w] = __shfl_up(gt[w], 1, 64);
+        gp[w] = tvd_lane_up(gt[w]);
+    }
+    if (lane >= 1 && lane <= TVD_XSEG64 && in && x >= pb.lo[0] && x < pb.lo[0] + pb.r[0]) {
+        double F[7];
+        tvd_flux_wave(W, uL, uR, a.cs, dtdx, dxdt, gm, gt, gp, ck, F);
+        tvd_store(a, c, F);
+    }
+}
+
+static __global__ __launch_bounds__(256, 2) void k_tvd_sweep_yz64(const BoxDesc* __restrict__ boxes, Plan plan,
+                                                           TvdSweepArgs<double> a) {
+    __shared__ double sg[6][256];
+    const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
+    const long long g0 = (long long)blk * 256;   // first item of this workgroup; total is a multiple of 256
+    int b = 0;
+    if (plan.nbox > 1) {
+        int lo = 0, hi = plan.nbox - 1;
+        while (lo < hi) {
+            int mid = (lo + hi + 1) >> 1;
+            if (plan.boxes[mid].start <= g0) lo = mid; else hi = mid - 1;
+        }
+        b = lo;
+    }
+    const PlanBox& pb = plan.boxes[b];
+    const int d = a.dir, ta = d == 1 ? 2 : 1;   // sweep axis, other transverse axis
+    const unsigned t = threadIdx.x, tx = t % TVD_X64, te = t / TVD_X64;
+    const unsigned len = (unsigned)pb.r[d] + 2u, nxt = ((unsigned)pb.r[0] + TVD_X64 - 1) / TVD_X64;
+    const unsigned cols = nxt * (unsigned)pb.r[ta];
+    const unsigned long long e0 = (unsigned long long)((g0 - pb.start) >> 8) * (TVD_ROWS64 - 2);
+    const unsigned col0 = (unsigned)(e0 / len), off = (unsigned)(e0 - (unsigned long long)col0 * len) + te;
+    const unsigned up = len >= TVD_ROWS64 ? (off >= len ? 1u : 0u) : off / len;
+    const unsigned col = col0 + up;
+    const int f = pb.lo[d] - 1 + (int)(off - up * len);   // this thread's face
+    unsigned xt = col0 % nxt + up, tr = col0 / nxt;
+    while (xt >= nxt) {
+        xt -= nxt;
+        tr++;
+    }
+    const int i = pb.lo[0] + (int)(xt * TVD_X64 + tx), it = pb.lo[ta] + (int)tr;
+    const bool in = col < cols && i < pb.lo[0] + pb.r[0];
+    const BoxDesc& B = boxes[b];
+    const long long s = tvd_stride(B, d);
+    const long long c = d == 1 ? cell_index(B, in ? i : pb.lo[0], in ? f : pb.lo[1], in ? it : pb.lo[2])
+                               : cell_index(B, in ? i : pb.lo[0], in ? it : pb.lo[1], in ? f : pb.lo[2]);
+    double dtdx, dxdt;
+    tvd_dts(a, B, b, dtdx, dxdt);
+    double uL[7], uR[7], ck[6], gt[6];
+    tvd_load(a, c, uL);
+    tvd_load(a, c + s, uR);
+    TvdWave<double> W;
+    tvd_eig_wave(uL, uR, a.cs, dtdx, W, gt, ck);
+#pragma unroll
+    for (int w = 0; w < 6; w++) sg[w][t] = gt[w];
+    __syncthreads();
+    if (te >= 1 && te < TVD_ROWS64 - 1 && in && f >= pb.lo[d] && f < pb.lo[d] + pb.r[d]) {
+        double gm[6], gp[6], F[7];
+#pragma unroll
+        for (int w = 0; w < 6; w++) {
+            gm[w] = sg[w][t - TVD_X64];
+            gp[w] = sg[w][t + TVD_X64];
+        }
+        tvd_flux_wave(W, uL, uR, a.cs, dtdx, dxdt, gm, gt, gp, ck, F);
+        tvd_store(a, c, F);
     }
 }
 
@@ -906,16 +1070,14 @@ void launch_tvd_flux(const Launch& L, const TvdSweepArgs<real>& a) {
 template <class real>
 void launch_tvd_sweep(const Launch& L, const TvdSweepArgs<real>& a) {
     if (L.plan.total <= 0) return;
-    if (a.dir == 0)
-        hipLaunchKernelGGL((k_tvd_sweep_x<real>), dim3(L.blocks()), dim3(256), 0, L.stream, L.boxes, L.plan, a);
-    else
-        hipLaunchKernelGGL((k_tvd_sweep_m<real>), dim3(L.blocks()), dim3(256), 0, L.stream, L.boxes, L.plan, a);
-}
-template <class real>
-int tvd_sweep_waves_per_cu() {
-    int n = 0;
-    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_tvd_sweep_m<real>, 256, 0);
-    return 4 * (e == hipSuccess && n > 0 ? n : 1);
+    const dim3 g(L.blocks()), n(256);
+    if constexpr (sizeof(real) == 8) {
+        if (a.dir == 0) hipLaunchKernelGGL(k_tvd_sweep_x64, g, n, 0, L.stream, L.boxes, L.plan, a);
+        else hipLaunchKernelGGL(k_tvd_sweep_yz64, g, n, 0, L.stream, L.boxes, L.plan, a);
+    } else {
+        if (a.dir == 0) hipLaunchKernelGGL((k_tvd_sweep_x<real>), g, n, 0, L.stream, L.boxes, L.plan, a);
+        else hipLaunchKernelGGL((k_tvd_sweep_m<real>), g, n, 0, L.stream, L.boxes, L.plan, a);
+    }
 }
 template <class real>
 void launch_tvd_hlle(const Launch& L, const TvdSweepArgs<real>& a) {
@@ -956,7 +1118,6 @@ void launch_tvd_max_speed(const Launch& L, const QPtrs<real>& q, double cs, unsi
     template void launch_tvd_eig<T>(const Launch&, const TvdSweepArgs<T>&);         \
     template void launch_tvd_flux<T>(const Launch&, const TvdSweepArgs<T>&);        \
     template void launch_tvd_sweep<T>(const Launch&, const TvdSweepArgs<T>&);       \
-    template int tvd_sweep_waves_per_cu<T>();                                       \
     template void launch_tvd_hlle<T>(const Launch&, const TvdSweepArgs<T>&);        \
     template void launch_tvd_corner<T>(const Launch&, const TvdCornerArgs<T>&);     \
     template void launch_tvd_center<T>(const Launch&, const TvdCenterArgs<T>&);     \
