@@ -17,7 +17,8 @@ template <class real>
 struct GhostArgs {
     real* r[7 + MAXPASS];
     double* d[3];
-    int nreal, ndbl, depth;
+    int nreal, depth;     // fields r[0 .. nreal) and d, to this depth
+    int nreal2, depth2;   // and r[nreal .. nreal2), the passives, to depth2 <= depth
 };
 
 template <class real>
@@ -120,7 +121,6 @@ template <class real> void launch_prot_flag(const Launch& L, const ProtArgs<real
 template <class real> void launch_prot_fix(const Launch& L, const ProtArgs<real>& a);
 
 template <class real> void launch_restore_shell(const Launch& L, const ShellArgs<real>& a);
-template <class real> void launch_fill_ghosts(const Launch& L, const GhostArgs<real>& a);
 template <class real> void launch_fill_ghost_band(const Launch& L, const GhostArgs<real>& a);
 template <class real> void launch_pass_stage(const Launch& L, const PassStageArgs<real>& a);
 template <class real> void launch_max_speed(const Launch& L, const QPtrs<real>& q, double cs, unsigned long long* cmax);

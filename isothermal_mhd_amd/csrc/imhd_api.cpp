@@ -137,7 +137,7 @@ struct imhd_ctx {
     size_t stage_n = 0;
     // plans
     PlanDev pl_pflux[3], pl_pcorner, pl_pupd, pl_cflux[3], pl_ccorner, pl_cupd;
-    PlanDev pl_gband, pl_pgband;
+    PlanDev pl_gband;
     PlanDev pl_ghost, pl_pghost, pl_int, pl_vel, pl_ppflux[3], pl_ppupd, pl_pcflux[3], pl_pfupd;
     PlanDev pl_pstage[2];   // fused passive stages (column plans when zseg > 0)
     PlanDev pl_teig_p[2][3], pl_tflux_p[3], pl_teig_c[2][3], pl_tflux_c[3];
@@ -341,8 +341,8 @@ int build_plan(imhd_ctx* c, PlanDev& p, int which, int dir, int seg = 0, bool tr
             pb.lo[a] = lo;
             pb.r[a] = std::max(0, hi - lo + 1);
         }
-        if (which == 14 || which == 15) {  // ghost band of depth w, enumerated linearly
-            long long w = which == 14 ? B.nb : 3;
+        if (which == 14) {  // ghost band of depth w, enumerated linearly
+            const long long w = B.nb;
             long long E0 = B.n[0] + 2 * w, E1 = B.n[1] + 2 * w;
             long long cnt = E0 * E1 * 2 * w + E0 * 2 * w * B.n[2] + 2 * w * (long long)B.n[1] * B.n[2];
             pb.lo[0] = pb.lo[1] = pb.lo[2] = 0;
@@ -1033,25 +1033,16 @@ void restore_shell(imhd_ctx* c) {
 template <class real>
 void fill_ghosts(imhd_ctx* c) {
     c->ghost_images = true;
-    {
-        ProfScope ps(c, "fill_ghosts", c->pl_gband.active);
-        GhostArgs<real> g{};
-        for (int f = 0; f < 7; f++) g.r[f] = R<real>(c->q[c->cur][f]);
-        for (int d = 0; d < 3; d++) g.d[d] = c->b[c->cur][d];
-        g.nreal = 7;
-        g.ndbl = 3;
-        g.depth = c->hb[0].nb;
-        launch_fill_ghost_band<real>(mk(c, c->pl_gband), g);
-    }
-    if (c->cfg.npass > 0) {
-        ProfScope ps(c, "fill_ghosts_pass", c->pl_pgband.active);
-        GhostArgs<real> g{};
-        for (int p = 0; p < c->cfg.npass; p++) g.r[p] = R<real>(c->qp[c->pcur][p]);
-        g.nreal = c->cfg.npass;
-        g.ndbl = 0;
-        g.depth = 3;
-        launch_fill_ghost_band<real>(mk(c, c->pl_pgband), g);
-    }
+    ProfScope ps(c, "fill_ghosts", c->pl_gband.active);
+    GhostArgs<real> g{};
+    for (int f = 0; f < 7; f++) g.r[f] = R<real>(c->q[c->cur][f]);
+    for (int d = 0; d < 3; d++) g.d[d] = c->b[c->cur][d];
+    for (int p = 0; p < c->cfg.npass; p++) g.r[7 + p] = R<real>(c->qp[c->pcur][p]);
+    g.nreal = 7;
+    g.depth = c->hb[0].nb;
+    g.nreal2 = 7 + c->cfg.npass;
+    g.depth2 = 3;   // passive_mod.f90:52
+    launch_fill_ghost_band<real>(mk(c, c->pl_gband), g);
 }
 
 template <class real>
@@ -2314,7 +2305,6 @@ int imhd_create_ensemble(const imhd_config* cfg, int nbox, imhd_ctx** out) {
     if ((rc = build_plan(c, c->pl_cupd, 5, -1, c->zseg))) return rc;
     if ((rc = build_plan(c, c->pl_ghost, 6, -1))) return rc;
     if ((rc = build_plan(c, c->pl_gband, 14, -1))) return rc;
-    if ((rc = build_plan(c, c->pl_pgband, 15, -1))) return rc;
     if ((rc = build_plan(c, c->pl_pghost, 7, -1))) return rc;
     if ((rc = build_plan(c, c->pl_int, 8, -1))) return rc;
     if ((rc = build_plan(c, c->pl_vel, 9, -1))) return rc;

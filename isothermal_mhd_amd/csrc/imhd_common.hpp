@@ -72,30 +72,65 @@ __device__ __forceinline__ unsigned floor_images(int n0, int n1, int n2, int i, 
     return along(i, n0) * along(j, n1) * along(k, n2);
 }
 
-// Maps this thread to (box, i, j, k).  Returns false for padding threads.
+// Item t of the 256 that begin at loc0, in an r0 x r1 x ... enumeration, x fastest.  loc0 is
+// the same for the whole workgroup, so its divisions are scalar and 32-bit; a lane adds its
+// own offset and carries it over the row ends it passes.  (Two 64-bit divisions per lane were
+// about 250 vector instructions before the first load.  FP32 200^3: half-step faces 0.157 ->
+// 0.125 ms, corner EMF 0.238 -> 0.211, passive corrector 0.227 -> 0.184.)
+__device__ __forceinline__ void item_xyz(unsigned long long loc0, unsigned t, unsigned r0, unsigned r1, unsigned& x,
+                                         unsigned& y, unsigned& z) {
+    unsigned row, x0;
+    if (loc0 >> 32 == 0) {
+        row = (unsigned)loc0 / r0;
+        x0 = (unsigned)loc0 - row * r0;
+    } else {
+        row = (unsigned)(loc0 / r0);
+        x0 = (unsigned)(loc0 - (unsigned long long)row * r0);
+    }
+    z = row / r1;
+    y = row - z * r1;
+    x = x0 + t;
+    if (r0 >= 64u) {   // x < r0 + 255: at most 4 rows passed
+#pragma unroll
+        for (int n = 0; n < 4; n++)
+            if (x >= r0) { x -= r0; y++; }
+    } else {
+        const unsigned up = x / r0;
+        x -= up * r0;
+        y += up;
+    }
+    if (y >= r1) {
+        const unsigned uz = y / r1;
+        y -= uz * r1;
+        z += uz;
+    }
+}
+
+// Maps this thread to (box, i, j, k), for workgroups of 256 threads (every box's items begin
+// at a multiple of 256, so a workgroup serves one box).  Returns false for padding threads.
 __device__ __forceinline__ bool plan_item(const Plan& p, int& box, int& i, int& j, int& k) {
-    unsigned blk = xcd_block(blockIdx.x, gridDim.x);
-    long long g = (long long)blk * blockDim.x + threadIdx.x;
+    const long long g0 = (long long)xcd_block(blockIdx.x, gridDim.x) * 256;
+    const long long g = g0 + threadIdx.x;
     if (g >= p.total) return false;
     int b = 0;
     if (p.nbox > 1) {
         int lo = 0, hi = p.nbox - 1;
         while (lo < hi) {
             int mid = (lo + hi + 1) >> 1;
-            if (p.boxes[mid].start <= g) lo = mid; else hi = mid - 1;
+            if (p.boxes[mid].start <= g0) lo = mid; else hi = mid - 1;
         }
         b = lo;
     }
     const PlanBox& pb = p.boxes[b];
-    long long loc = g - pb.start;
+    const long long loc = g - pb.start;
     const long long r0 = pb.r[0], r1 = pb.r[1], r2 = pb.r[2];
     if (loc >= r0 * r1 * r2) return false;
-    long long t = loc / r0;
-    i = pb.lo[0] + (int)(loc - t * r0);
     const long long sy = p.sy;
     if (sy > 0 && r1 > sy) {
         // y-strip order: strip s holds rows [s sy, (s+1) sy) of every k, k outer within it,
         // so a strip's k-1 / k+1 planes stay in the XCD's L2 while the strip is swept
+        const long long t = loc / r0;
+        i = pb.lo[0] + (int)(loc - t * r0);
         const long long full = r1 / sy, per = sy * r2;
         const long long s = t / per;
         long long jj, kk;
@@ -111,9 +146,11 @@ __device__ __forceinline__ bool plan_item(const Plan& p, int& box, int& i, int& 
         j = pb.lo[1] + (int)jj;
         k = pb.lo[2] + (int)kk;
     } else {
-        long long u = t / r1;
-        j = pb.lo[1] + (int)(t - u * r1);
-        k = pb.lo[2] + (int)u;
+        unsigned x, y, z;
+        item_xyz((unsigned long long)(g0 - pb.start), threadIdx.x, (unsigned)pb.r[0], (unsigned)pb.r[1], x, y, z);
+        i = pb.lo[0] + (int)x;
+        j = pb.lo[1] + (int)y;
+        k = pb.lo[2] + (int)z;
     }
     box = b;
     return true;
@@ -133,12 +170,11 @@ __device__ __forceinline__ bool plan_item_box(const Plan& p, int& box, int& i, i
     box = 0;
     bool act = plan_item(p, box, i, j, k);
     if (!act && p.nbox > 1) {
-        unsigned blk = xcd_block(blockIdx.x, gridDim.x);
-        long long g = (long long)blk * blockDim.x + threadIdx.x;
+        const long long g0 = (long long)xcd_block(blockIdx.x, gridDim.x) * 256;
         int lo = 0, hi = p.nbox - 1;
         while (lo < hi) {
             int mid = (lo + hi + 1) >> 1;
-            if (p.boxes[mid].start <= g) lo = mid; else hi = mid - 1;
+            if (p.boxes[mid].start <= g0) lo = mid; else hi = mid - 1;
         }
         box = lo;
     }

@@ -422,27 +422,23 @@ __global__ __launch_bounds__(256) void k_tvd_sweep_x(const BoxDesc* __restrict__
 template <class real>
 __global__ __launch_bounds__(256, 1) void k_tvd_sweep_m(const BoxDesc* __restrict__ boxes, Plan plan,
                                                                               TvdSweepArgs<real> a) {
-    const unsigned blk = xcd_block(blockIdx.x, gridDim.x);
-    const long long g = (long long)blk * blockDim.x + threadIdx.x;
-    if (g >= plan.total) return;
+    const long long w0 = (long long)xcd_block(blockIdx.x, gridDim.x) * 256;   // a workgroup serves one box
+    if (w0 + threadIdx.x >= plan.total) return;
     int b = 0;
     if (plan.nbox > 1) {
         int lo = 0, hi = plan.nbox - 1;
         while (lo < hi) {
             int mid = (lo + hi + 1) >> 1;
-            if (plan.boxes[mid].start <= g) lo = mid; else hi = mid - 1;
+            if (plan.boxes[mid].start <= w0) lo = mid; else hi = mid - 1;
         }
         b = lo;
     }
     const PlanBox& pb = plan.boxes[b];
     const int d = a.dir, ta = d == 1 ? 2 : 1;   // sweep axis, other transverse axis
-    const long long loc = g - pb.start;
-    const long long cols = (long long)pb.r[0] * pb.r[ta];
-    if (loc >= cols * pb.zn) return;
-    const int i = pb.lo[0] + (int)(loc % pb.r[0]);
-    const long long t = loc / pb.r[0];
-    const int it = pb.lo[ta] + (int)(t % pb.r[ta]);
-    const int sgi = (int)(t / pb.r[ta]);
+    if (w0 + threadIdx.x - pb.start >= (long long)pb.r[0] * pb.r[ta] * pb.zn) return;
+    unsigned xi, ti, si;
+    item_xyz((unsigned long long)(w0 - pb.start), threadIdx.x, (unsigned)pb.r[0], (unsigned)pb.r[ta], xi, ti, si);
+    const int i = pb.lo[0] + (int)xi, it = pb.lo[ta] + (int)ti, sgi = (int)si;
     const int f0 = pb.lo[d] + sgi * pb.seg;
     const int f1 = min(f0 + pb.seg - 1, pb.lo[d] + pb.r[d] - 1);
     const BoxDesc& B = boxes[b];
