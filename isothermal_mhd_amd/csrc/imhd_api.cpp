@@ -106,8 +106,10 @@ struct imhd_ctx {
     bool fft_have_plan = false;
     int fft_n = 0;
     unsigned long long fft_bytes = 0;   // plan work area and buffers (in dev_bytes too)
-    void* fft_in = nullptr;         // n^3 floats (packed field)
-    void* fft_out[3] = {};          // n^2 (n/2+1) complex each (mode decomposition uses 3)
+    // n^2 (n/2+1) complex each: packed components (n^3 floats) and transforms.  A density
+    // spectrum uses fft_in and fft_out[0], everything else all four
+    void* fft_in = nullptr;
+    void* fft_out[3] = {};
     void* fft_acc = nullptr;        // (n/2)^3 floats (octant power)
     void* fft_bins = nullptr;       // 8 n doubles (bins) + 3 (mean field)
     // OU forcing of the native loop
@@ -1987,7 +1989,7 @@ static int fft_setup(imhd_ctx* c, int n, int nout) {
         HIPCK(c, hipStreamSynchronize(c->st));
         fft_release(c);
         const int h = n / 2;
-        const long long nc = (long long)n * n * n, no = (long long)h * h * h;
+        const long long nk = (long long)n * n * (h + 1), no = (long long)h * h * h;
         size_t work = 0;
         if (hipfftPlan3d(&c->fft_plan, n, n, n, HIPFFT_R2C) != HIPFFT_SUCCESS) FAIL(c, IMHD_EHIP, "hipfftPlan3d failed");
         c->fft_have_plan = true;
@@ -1997,7 +1999,7 @@ static int fft_setup(imhd_ctx* c, int n, int nout) {
         }
         c->fft_bytes += work;
         c->dev_bytes += work;
-        if ((rc = fft_malloc(c, &c->fft_in, (size_t)nc * 4)) || (rc = fft_malloc(c, &c->fft_acc, (size_t)no * 4)) ||
+        if ((rc = fft_malloc(c, &c->fft_in, (size_t)nk * 8)) || (rc = fft_malloc(c, &c->fft_acc, (size_t)no * 4)) ||
             (rc = fft_malloc(c, &c->fft_bins, (size_t)(8 * n + 3) * 8))) {
             fft_release(c);
             return rc;
@@ -2022,21 +2024,33 @@ template <class real>
 static int spectrum_t(imhd_ctx* c, int bx, int which, double* k_out, double* pk_out) {
     const BoxDesc& B = c->hb[bx];
     const int n = B.n[0], h = n / 2;
+    const int ncomp = which == SPEC_DENSITY ? 1 : 3;
     int rc = fft_setup(c, n, 1);
     if (rc) return rc;
+    // three components are packed in one pass where there is ample room for them: in fft_in and
+    // the last two transform buffers (at most a quarter of the free memory, if they have yet
+    // to be made), the transforms one after the other in the first
+    bool together = ncomp == 3 && !getenv("IMHD_TEST_SPEC_SINGLE");   // tests: as if there were no room
+    if (together && !(c->fft_out[1] && c->fft_out[2])) {
+        size_t room = 0, total = 0;
+        together = hipMemGetInfo(&room, &total) == hipSuccess &&
+                   2 * ((size_t)n * n * (h + 1) * 8) <= room / 4 && fft_setup(c, n, 3) == IMHD_OK;
+        if (!together) (void)hipGetLastError();
+    }
     struct Raw { double* p; };   // the cached buffers, in the form the launch calls take
-    const Raw fin{(double*)c->fft_in}, fout{(double*)c->fft_out[0]}, acc{(double*)c->fft_acc},
-        pk{(double*)c->fft_bins};
+    const Raw fout{(double*)c->fft_out[0]}, acc{(double*)c->fft_acc}, pk{(double*)c->fft_bins};
     const hipfftHandle plan = c->fft_plan;
     SpecPackArgs<real> a{};
     for (int f = 0; f < 7; f++) a.q[f] = R<real>(c->q[c->cur][f]);
     a.which = which;
-    a.out = (float*)fin.p;
-    const int ncomp = which == SPEC_DENSITY ? 1 : 3;
+    float* const in[3] = {(float*)c->fft_in, (float*)(together ? c->fft_out[1] : c->fft_in),
+                          (float*)(together ? c->fft_out[2] : c->fft_in)};
     for (int comp = 0; comp < ncomp; comp++) {
-        a.comp = comp;
-        launch_spec_pack<real>(c->st, B, a);
-        if (hipfftExecR2C(plan, (hipfftReal*)fin.p, (hipfftComplex*)fout.p) != HIPFFT_SUCCESS)
+        if (comp == 0 || !together) {
+            for (int d = 0; d < 3; d++) a.out[d] = (together || d == comp) ? in[d] : nullptr;
+            launch_spec_pack<real>(c->st, B, a);
+        }
+        if (hipfftExecR2C(plan, (hipfftReal*)in[comp], (hipfftComplex*)fout.p) != HIPFFT_SUCCESS)
             FAIL(c, IMHD_EHIP, "hipfftExecR2C failed");
         launch_spec_accum(c->st, (const float*)fout.p, n, (float*)acc.p, comp == 0);
     }
@@ -2066,20 +2080,20 @@ static int mode_spectra_t(imhd_ctx* c, int bx, double* k_out, double* P_out) {
     int rc = fft_setup(c, n, 3);
     if (rc) return rc;
     struct Raw { double* p; };
-    const Raw fin{(double*)c->fft_in},
-        f[3] = {{(double*)c->fft_out[0]}, {(double*)c->fft_out[1]}, {(double*)c->fft_out[2]}},
-        P{(double*)c->fft_bins}, b0{(double*)c->fft_bins + 8 * n};
+    const Raw P{(double*)c->fft_bins}, b0{(double*)c->fft_bins + 8 * n};
     const hipfftHandle plan = c->fft_plan;
     SpecPackArgs<real> a{};
     for (int q = 0; q < 7; q++) a.q[q] = R<real>(c->q[c->cur][q]);
     a.which = SPEC_VPERP;
-    a.out = (float*)fin.p;
-    for (int d = 0; d < 3; d++) {
-        a.comp = d;
-        launch_spec_pack<real>(c->st, B, a);
-        if (hipfftExecR2C(plan, (hipfftReal*)fin.p, (hipfftComplex*)f[d].p) != HIPFFT_SUCCESS)
+    // packed components in three of the four buffers; each transform goes to the buffer
+    // that the one before has freed
+    void* const in[3] = {c->fft_in, c->fft_out[1], c->fft_out[2]};
+    const Raw f[3] = {{(double*)c->fft_out[0]}, {(double*)c->fft_in}, {(double*)c->fft_out[1]}};
+    for (int d = 0; d < 3; d++) a.out[d] = (float*)in[d];
+    launch_spec_pack<real>(c->st, B, a);
+    for (int d = 0; d < 3; d++)
+        if (hipfftExecR2C(plan, (hipfftReal*)in[d], (hipfftComplex*)f[d].p) != HIPFFT_SUCCESS)
             FAIL(c, IMHD_EHIP, "hipfftExecR2C failed");
-    }
     launch_reset_u64(c->st, (unsigned long long*)b0.p, 3);
     launch_mean_b<real>(c->st, B, R<real>(c->q[c->cur][4]), R<real>(c->q[c->cur][5]), R<real>(c->q[c->cur][6]), b0.p);
     const float k0 = (float)(8.0 * atan(1.0));

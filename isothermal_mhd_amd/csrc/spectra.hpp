@@ -12,8 +12,8 @@ enum { SPEC_DENSITY = 0, SPEC_VELOCITY = 1, SPEC_BFIELD = 2, SPEC_VPAR = 3, SPEC
 template <class real>
 struct SpecPackArgs {
     const real* q[7];
-    int which, comp;   // field kind, component 0..2
-    float* out;        // n0 x n1 x n2 interior, x fastest
+    int which;         // field kind
+    float* out[3];     // its components (density: out[0]), n0 x n1 x n2 interior, x fastest; null: not formed
 };
 
 template <class real>
