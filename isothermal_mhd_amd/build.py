@@ -12,6 +12,7 @@ OBJ = os.path.join(HERE, "_build")
 # (source, extra flags): the FP32 kernels may contract to FMA; everything else may not.
 SOURCES = [("vl_kernels_f64.hip", ["-ffp-contract=off"]),
            ("vl_kernels_f32.hip", ["-ffp-contract=fast"]),
+           ("vl_near_f64.hip", ["-ffp-contract=off"]),
            ("vl_char_f64.hip", ["-ffp-contract=off"]),
            ("tvd_kernels_f64.hip", ["-ffp-contract=off"]),
            ("tvd_kernels_f32.hip", ["-ffp-contract=fast"]),

@@ -148,6 +148,11 @@ void launch_vl_stage(hipStream_t st, const BoxDesc* boxes, const TilePlan& plan,
 // workgroups of a fused stage resident per CU (occupancy of the kernel as compiled)
 template <class real, int RS>
 int vl_stage_blocks_per_cu(int kind, int shape);
+// kinds 0 (PRED) and 1 in FP64: k_vl_near, neighbours shared through LDS and lane shifts
+template <int RS, bool PRED>
+void launch_vl_near(hipStream_t st, const BoxDesc* boxes, const TilePlan& plan, const StageArgs<double>& a, int shape);
+template <int RS, bool PRED>
+int vl_near_blocks_per_cu(int shape);
 // kind 3 in FP64: k_vl_char, each cell's edge values formed once (tile shapes 0 and 1)
 template <int RS>
 void launch_vl_char(hipStream_t st, const BoxDesc* boxes, const TilePlan& plan, const StageArgs<double>& a, int shape);

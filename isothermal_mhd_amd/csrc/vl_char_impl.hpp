@@ -40,13 +40,6 @@
 
 namespace imhd {
 
-__device__ __forceinline__ double lane_next_d(double x) {   // the value of lane l + 1
-    const long long v = __double_as_longlong(x);
-    const int lo = __builtin_amdgcn_mov_dpp((int)(unsigned)v, 0x130, 0xf, 0xf, true);
-    const int hi = __builtin_amdgcn_mov_dpp((int)(v >> 32), 0x130, 0xf, 0xf, true);
-    return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
-}
-
 // E(c) from W[0..3] = cells c-1 .. c+2 and the cell's upper face field: the values of
 // prim_eigvecs and char_delw bit for bit, formed a wave pair at a time so that few are live.
 // The two waves of a pair have eigenvectors that differ in signs only; a product's sign is

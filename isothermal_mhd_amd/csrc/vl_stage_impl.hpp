@@ -75,8 +75,7 @@ __device__ __forceinline__ real stage_face_own(const SweepArgs<real>& a, const r
     }
 }
 // z face k+1/2: predictor between the thread's own cells of planes k (UL) and k+1 (UR),
-// both in registers; FP64 corrector with those two of its four stencil cells from
-// registers; FP32 corrector as above (holding them spills at 128 VGPRs).
+// both in registers; correctors load their stencils (holding them spills at 128 VGPRs).
 template <class real, int RS, int KIND>
 __device__ __forceinline__ real stage_face_z(const SweepArgs<real>& a, const real* UL, const real* UR, long long c,
                                              long long s, real* F) {
@@ -95,14 +94,6 @@ __device__ __forceinline__ real stage_face_z(const SweepArgs<real>& a, const rea
         return smax;
     } else if constexpr (KIND >= 2) {
         return ppm_flux_calc<real, RS, KIND == 3>(a, c, s, F);
-    } else if constexpr (sizeof(real) == 8) {
-        // FP64 (2 waves per SIMD, registers to spare): planes k and k+1 from registers
-        real W[4][6];
-        prim_load(a, c - s, W[0]);
-        prim_rot(UL[0], UL[perm(2, 1)], UL[perm(2, 2)], UL[perm(2, 3)], UL[perm(2, 5)], UL[perm(2, 6)], W[1]);
-        prim_rot(UR[0], UR[perm(2, 1)], UR[perm(2, 2)], UR[perm(2, 3)], UR[perm(2, 5)], UR[perm(2, 6)], W[2]);
-        prim_load(a, c + 2 * s, W[3]);
-        return plm_flux<real, RS>(a, W, bn_at(a, c), F);
     } else {
         return flux_corr_calc<real, RS>(a, c, s, F);
     }
@@ -123,6 +114,13 @@ __device__ __forceinline__ double lane_prev_d(double x) {
     const long long v = __double_as_longlong(x);
     const int lo = __builtin_amdgcn_mov_dpp((int)(unsigned)v, 0x138, 0xf, 0xf, true);
     const int hi = __builtin_amdgcn_mov_dpp((int)(v >> 32), 0x138, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
+}
+
+__device__ __forceinline__ double lane_next_d(double x) {
+    const long long v = __double_as_longlong(x);
+    const int lo = __builtin_amdgcn_mov_dpp((int)(unsigned)v, 0x130, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(v >> 32), 0x130, 0xf, 0xf, true);
     return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
 
@@ -857,8 +855,9 @@ __global__ __launch_bounds__(TX * TY, VS_WAVES) void k_vl_stage(const BoxDesc* _
     if (!PRED && a.cmax != nullptr) atomic_max_nonneg(a.cmax, b, (double)cfl);
 }
 
-// kind: 0 predictor, 1 PLM corrector, 2 PPM-primitive corrector, 3 PPM-characteristic
-// corrector (FP32; FP64 runs k_vl_char); shape 2 exists in FP32 only
+// kind: 0 predictor, 1 PLM corrector (both FP32; FP64 runs k_vl_near), 2 PPM-primitive
+// corrector, 3 PPM-characteristic corrector (FP32; FP64 runs k_vl_char); shape 2 exists in
+// FP32 only
 template <class real, int RS, int KIND>
 void launch_vl_stage_k(hipStream_t st, const BoxDesc* boxes, const TilePlan& plan, const StageArgs<real>& a,
                        int shape) {
@@ -897,19 +896,22 @@ int vl_stage_blocks_per_cu_k(int shape) {
 }
 template <class real, int RS>
 int vl_stage_blocks_per_cu(int kind, int shape) {
-    switch (kind) {
-        case 0: return vl_stage_blocks_per_cu_k<real, RS, 0>(shape);
-        case 1: return vl_stage_blocks_per_cu_k<real, RS, 1>(shape);
-        case 2: return vl_stage_blocks_per_cu_k<real, RS, 2>(shape);
-        case 4:
-            if constexpr (sizeof(real) == 4) return vl_stage_blocks_per_cu_k<real, RS, 4>(shape);
-            return vl_stage_blocks_per_cu_k<real, RS, 1>(shape);
-        case 5:
-            if constexpr (sizeof(real) == 4) return vl_stage_blocks_per_cu_k<real, RS, 5>(shape);
-            return vl_stage_blocks_per_cu_k<real, RS, 0>(shape);
-        default:
-            if constexpr (sizeof(real) == 4) return vl_stage_blocks_per_cu_k<real, RS, 3>(shape);
-            return vl_char_blocks_per_cu<RS>(shape);
+    if constexpr (sizeof(real) == 8) {
+        switch (kind) {
+            case 0: return vl_near_blocks_per_cu<RS, true>(shape);
+            case 1: return vl_near_blocks_per_cu<RS, false>(shape);
+            case 2: return vl_stage_blocks_per_cu_k<real, RS, 2>(shape);
+            default: return vl_char_blocks_per_cu<RS>(shape);
+        }
+    } else {
+        switch (kind) {
+            case 0: return vl_stage_blocks_per_cu_k<real, RS, 0>(shape);
+            case 1: return vl_stage_blocks_per_cu_k<real, RS, 1>(shape);
+            case 2: return vl_stage_blocks_per_cu_k<real, RS, 2>(shape);
+            case 4: return vl_stage_blocks_per_cu_k<real, RS, 4>(shape);
+            case 5: return vl_stage_blocks_per_cu_k<real, RS, 5>(shape);
+            default: return vl_stage_blocks_per_cu_k<real, RS, 3>(shape);
+        }
     }
 }
 
@@ -917,22 +919,22 @@ template <class real, int RS>
 void launch_vl_stage(hipStream_t st, const BoxDesc* boxes, const TilePlan& plan, const StageArgs<real>& a, int kind,
                      int shape) {
     if (plan.total <= 0) return;
-    switch (kind) {
-        case 0: launch_vl_stage_k<real, RS, 0>(st, boxes, plan, a, shape); break;
-        case 1: launch_vl_stage_k<real, RS, 1>(st, boxes, plan, a, shape); break;
-        case 2: launch_vl_stage_k<real, RS, 2>(st, boxes, plan, a, shape); break;
-        case 4:   // FP32 only; an FP64 context runs the PLM corrector as kind 1
-            if constexpr (sizeof(real) == 4) launch_vl_stage_k<real, RS, 4>(st, boxes, plan, a, shape);
-            else launch_vl_stage_k<real, RS, 1>(st, boxes, plan, a, shape);
-            break;
-        case 5:   // FP32 only; an FP64 context runs the predictor as kind 0
-            if constexpr (sizeof(real) == 4) launch_vl_stage_k<real, RS, 5>(st, boxes, plan, a, shape);
-            else launch_vl_stage_k<real, RS, 0>(st, boxes, plan, a, shape);
-            break;
-        default:   // FP64 shares each cell's edge values between its faces
-            if constexpr (sizeof(real) == 4) launch_vl_stage_k<real, RS, 3>(st, boxes, plan, a, shape);
-            else launch_vl_char<RS>(st, boxes, plan, a, shape);
-            break;
+    if constexpr (sizeof(real) == 8) {
+        switch (kind) {
+            case 0: launch_vl_near<RS, true>(st, boxes, plan, a, shape); break;
+            case 1: launch_vl_near<RS, false>(st, boxes, plan, a, shape); break;
+            case 2: launch_vl_stage_k<real, RS, 2>(st, boxes, plan, a, shape); break;
+            default: launch_vl_char<RS>(st, boxes, plan, a, shape); break;
+        }
+    } else {
+        switch (kind) {
+            case 0: launch_vl_stage_k<real, RS, 0>(st, boxes, plan, a, shape); break;
+            case 1: launch_vl_stage_k<real, RS, 1>(st, boxes, plan, a, shape); break;
+            case 2: launch_vl_stage_k<real, RS, 2>(st, boxes, plan, a, shape); break;
+            case 4: launch_vl_stage_k<real, RS, 4>(st, boxes, plan, a, shape); break;
+            case 5: launch_vl_stage_k<real, RS, 5>(st, boxes, plan, a, shape); break;
+            default: launch_vl_stage_k<real, RS, 3>(st, boxes, plan, a, shape); break;
+        }
     }
 }
 
