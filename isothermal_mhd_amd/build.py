@@ -14,6 +14,7 @@ SOURCES = [("vl_kernels_f64.hip", ["-ffp-contract=off"]),
            ("vl_kernels_f32.hip", ["-ffp-contract=fast"]),
            ("vl_near_f64.hip", ["-ffp-contract=off"]),
            ("vl_char_f64.hip", ["-ffp-contract=off"]),
+           ("vl_char_f32.hip", ["-ffp-contract=fast-honor-pragmas"]),
            ("tvd_kernels_f64.hip", ["-ffp-contract=off"]),
            ("tvd_kernels_f32.hip", ["-ffp-contract=fast"]),
            ("aux_kernels.hip", ["-ffp-contract=off"]),

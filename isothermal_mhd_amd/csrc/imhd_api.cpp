@@ -421,7 +421,11 @@ int stage_kind(const imhd_ctx* c, bool corr) {
     if (c->prec == 32 && c->vsh) return k == 1 ? 4 : (k == 0 ? 5 : k);
     return k;
 }
-int stage_shape(const imhd_ctx* c, bool corr) { return corr ? c->vshape_c : c->vshape; }
+// (the characteristic PPM corrector has no 32 x 32 tiles: they would need 175 KB of LDS)
+int stage_shape(const imhd_ctx* c, bool corr) {
+    if (corr && stage_kind(c, true) == 3) return std::min(c->vshape_c, 1);
+    return corr ? c->vshape_c : c->vshape;
+}
 
 template <class real>
 int stage_blocks_per_cu(const imhd_ctx* c, bool corr) {
@@ -2183,6 +2187,9 @@ int imhd_create_ensemble(const imhd_config* cfg, int nbox, imhd_ctx** out) {
     }
     if (const char* e = getenv("IMHD_VSH")) c->vsh = atoi(e) != 0;
     c->vshape_c = c->vshape;
+    // FP32 characteristic PPM corrector: three 16 x 16 workgroups per CU (256^3: 2.76 ms; one
+    // of 32 x 16, which is all that the LDS holds, 2.97)
+    if (vs_kind(true, g.recon) == 3 && getenv("IMHD_VSHAPE") == nullptr) c->vshape_c = 0;
     if (const char* e = getenv("IMHD_VSHAPE_C")) {   // the corrector's alone
         const int v = std::min(VS_SHAPES - 1, std::max(0, atoi(e)));
         if (vs_shape_ok(g.precision, v)) c->vshape_c = v;

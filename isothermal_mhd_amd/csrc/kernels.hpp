@@ -153,10 +153,10 @@ template <int RS, bool PRED>
 void launch_vl_near(hipStream_t st, const BoxDesc* boxes, const TilePlan& plan, const StageArgs<double>& a, int shape);
 template <int RS, bool PRED>
 int vl_near_blocks_per_cu(int shape);
-// kind 3 in FP64: k_vl_char, each cell's edge values formed once (tile shapes 0 and 1)
-template <int RS>
-void launch_vl_char(hipStream_t st, const BoxDesc* boxes, const TilePlan& plan, const StageArgs<double>& a, int shape);
-template <int RS>
+// kind 3: k_vl_char, each cell's edge values formed once (tile shapes 0 and 1)
+template <class real, int RS>
+void launch_vl_char(hipStream_t st, const BoxDesc* boxes, const TilePlan& plan, const StageArgs<real>& a, int shape);
+template <class real, int RS>
 int vl_char_blocks_per_cu(int shape);
 constexpr int vs_kind(bool corrector, int recon) { return corrector ? 1 + recon : 0; }
 

@@ -19,10 +19,18 @@ __device__ __forceinline__ real fast_speed(const real* u, real asqr) {  // vanle
     return fsqrt(real(0.5) * (tmp1 + tmp2));
 }
 
-template <class real>
+// rho (v_n^2 + c^2) + (B_t^2 - B_n^2) / 2.  In FP32 the compiler may fuse either product into
+// the sum; PROD: the first one is rounded
+template <class real, bool PROD>
+__device__ __forceinline__ real normal_momentum_flux(real p, real pm) {
+    if constexpr (PROD && sizeof(real) == 4) return __builtin_fmaf(0.5f, pm, p);
+    else return p + real(0.5) * pm;
+}
+
+template <class real, bool PROD = false>
 __device__ __forceinline__ void phys_flux(const real* u, real asqr, real vx, real vy, real vz, real* F) {
     F[0] = u[1];
-    F[1] = u[0] * (vx * vx + asqr) + real(0.5) * (u[5] * u[5] + u[6] * u[6] - u[4] * u[4]);
+    F[1] = normal_momentum_flux<real, PROD>(u[0] * (vx * vx + asqr), u[5] * u[5] + u[6] * u[6] - u[4] * u[4]);
     F[2] = u[1] * vy - u[4] * u[5];
     F[3] = u[1] * vz - u[4] * u[6];
     F[4] = real(0);
@@ -31,7 +39,7 @@ __device__ __forceinline__ void phys_flux(const real* u, real asqr, real vx, rea
 }
 
 // HLLE with Einfeldt-type speeds clamped with 0 (vanleer_mod.f90:2867-2981)
-template <class real, bool VGIVEN = false>
+template <class real, bool VGIVEN = false, bool PROD = false>
 __device__ __forceinline__ void hlle(const real* uL, const real* uR, real asqr, real* F, real& smax,
                                      const real* vl = nullptr, const real* vr = nullptr) {
     real uavg[7], FL[7], FR[7];
@@ -45,8 +53,8 @@ __device__ __forceinline__ void hlle(const real* uL, const real* uR, real asqr, 
         vxL = fdiv(uL[1], uL[0]); vyL = fdiv(uL[2], uL[0]); vzL = fdiv(uL[3], uL[0]);
         vxR = fdiv(uR[1], uR[0]); vyR = fdiv(uR[2], uR[0]); vzR = fdiv(uR[3], uR[0]);
     }
-    phys_flux(uL, asqr, vxL, vyL, vzL, FL);
-    phys_flux(uR, asqr, vxR, vyR, vzR, FR);
+    phys_flux<real, PROD>(uL, asqr, vxL, vyL, vzL, FL);
+    phys_flux<real, PROD>(uR, asqr, vxR, vyR, vzR, FR);
     real cfL = fast_speed(uL, asqr), cfR = fast_speed(uR, asqr), cfa = fast_speed(uavg, asqr);
     real vxa = fdiv(uavg[1], uavg[0]);
     real sL = min3(vxL - cfL, vxa - cfa, real(0));
@@ -61,7 +69,7 @@ __device__ __forceinline__ void hlle(const real* uL, const real* uR, real asqr, 
 // VGIVEN: the caller passes the states' velocities (vl, vr) instead of having the momenta
 // divided by rho here (FP32 PLM: those it formed the momenta from; FP64 predictor: the cells'
 // own, divided once per cell instead of once per face and side).
-template <class real, bool VGIVEN = false>
+template <class real, bool VGIVEN = false, bool PROD = false>
 __device__ __forceinline__ void hlld(const real* uL, const real* uR, real asqr, real* F, real& smax,
                                      const real* vl = nullptr, const real* vr = nullptr) {
     real uavg[7], FL[7], FR[7];
@@ -77,8 +85,8 @@ __device__ __forceinline__ void hlld(const real* uL, const real* uR, real asqr, 
         vxL = fdiv(uL[1], uL[0]); vyL = fdiv(uL[2], uL[0]); vzL = fdiv(uL[3], uL[0]);
         vxR = fdiv(uR[1], uR[0]); vyR = fdiv(uR[2], uR[0]); vzR = fdiv(uR[3], uR[0]);
     }
-    phys_flux(uL, asqr, vxL, vyL, vzL, FL);
-    phys_flux(uR, asqr, vxR, vyR, vzR, FR);
+    phys_flux<real, PROD>(uL, asqr, vxL, vyL, vzL, FL);
+    phys_flux<real, PROD>(uR, asqr, vxR, vyR, vzR, FR);
     real cfL = fast_speed(uL, asqr), cfR = fast_speed(uR, asqr), cfa = fast_speed(uavg, asqr);
     real vxa = fdiv(uavg[1], uavg[0]);
     real sL = min3(vxL - cfL, vxa - cfa, real(0));
@@ -171,7 +179,7 @@ __device__ __forceinline__ void hlld(const real* uL, const real* uR, real asqr, 
 
 // Roe flux with arithmetic-mean state, K98 eigenvectors ("MODIFIED V1" degeneracy rules)
 // and the reference's Harten-type entropy fix, vanleer_mod.f90:2264-2863.
-template <class real>
+template <class real, bool PROD = false>
 __device__ __forceinline__ void roe(const real* qL, const real* qR, real cs, real* F, real& smax) {
     const real asqr = cs * cs;
     const real zero = real(ZERO);
@@ -279,7 +287,7 @@ __device__ __forceinline__ void roe(const real* qL, const real* qR, real cs, rea
     {
         real rho = qL[0], vx = fdiv(qL[1], rho), vy = fdiv(qL[2], rho), vz = fdiv(qL[3], rho), Bxx = qL[4], By = qL[5], Bz = qL[6];
         FLc[0] = rho * vx;
-        FLc[1] = rho * (vx * vx + cs * cs) + real(0.5) * (By * By + Bz * Bz - Bxx * Bxx);
+        FLc[1] = normal_momentum_flux<real, PROD>(rho * (vx * vx + cs * cs), By * By + Bz * Bz - Bxx * Bxx);
         FLc[2] = rho * vx * vy - Bxx * By;
         FLc[3] = rho * vx * vz - Bxx * Bz;
         FLc[4] = vx * By - vy * Bxx;
@@ -288,7 +296,7 @@ __device__ __forceinline__ void roe(const real* qL, const real* qR, real cs, rea
     {
         real rho = qR[0], vx = fdiv(qR[1], rho), vy = fdiv(qR[2], rho), vz = fdiv(qR[3], rho), Bxx = qR[4], By = qR[5], Bz = qR[6];
         FRc[0] = rho * vx;
-        FRc[1] = rho * (vx * vx + cs * cs) + real(0.5) * (By * By + Bz * Bz - Bxx * Bxx);
+        FRc[1] = normal_momentum_flux<real, PROD>(rho * (vx * vx + cs * cs), By * By + Bz * Bz - Bxx * Bxx);
         FRc[2] = rho * vx * vy - Bxx * By;
         FRc[3] = rho * vx * vz - Bxx * Bz;
         FRc[4] = vx * By - vy * Bxx;

@@ -4,7 +4,7 @@
 #include "vl_char_impl.hpp"
 
 namespace imhd {
-IMHD_INST_CHAR(RS_ROE)
-IMHD_INST_CHAR(RS_HLLD)
-IMHD_INST_CHAR(RS_HLLE)
+IMHD_INST_CHAR(double, RS_ROE)
+IMHD_INST_CHAR(double, RS_HLLD)
+IMHD_INST_CHAR(double, RS_HLLE)
 }  // namespace imhd

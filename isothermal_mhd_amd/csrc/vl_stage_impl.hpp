@@ -28,16 +28,13 @@ namespace imhd {
 
 // waves per SIMD the register allocation must allow: in FP32 the LDS of a 16 x 16 tile
 // (40 KB) fits 4 workgroups per CU and that of a 32 x 16 tile (80 KB) 2, 16 waves per CU
-// either way; FP64 needs more of both and gets 2 waves per SIMD; the characteristic PPM
-// corrector (KIND 3: six-cell stencils and 6 x 6 eigenvector matrices, about 210
-// registers) gets 2 in FP32 too, rather than spill at 128; the shared-slope PLM corrector
+// either way; FP64 needs more of both and gets 1; the shared-slope PLM corrector
 // (KIND 4) gets 3 on 16 x 16 tiles (three workgroups per CU) and 4 otherwise
 template <class real, int KIND, int N>
 constexpr int vs_waves() {
     if constexpr (sizeof(real) == 8) return 1;
     if constexpr (KIND == 4) return N == 256 ? 3 : 4;   // 16 x 16: 168 registers, three workgroups per CU
-    if constexpr (KIND == 5) return 4;
-    return KIND == 3 ? 2 : 4;
+    return 4;
 }
 #define VS_WAVES (vs_waves<real, KIND, TX * TY>())
 
@@ -45,8 +42,8 @@ constexpr int vs_waves() {
 // the thread's own, held in registers in the global field order, and only the neighbour is
 // loaded (same arithmetic as flux_pred_calc).  PLM corrector (KIND 1): flux_corr_calc's
 // arithmetic with the own cell from registers and the other three of its four-cell
-// stencil loaded.  PPM correctors (KIND 2 primitive, 3 characteristic): ppm_flux_calc,
-// which loads its six-cell stencil.
+// stencil loaded.  Primitive PPM corrector (KIND 2): ppm_flux_calc, which loads its six-cell
+// stencil.
 template <class real, int RS, int KIND, int D>
 __device__ __forceinline__ real stage_face_own(const SweepArgs<real>& a, const real* U, long long c, long long s,
                                                real* F) {
@@ -71,7 +68,7 @@ __device__ __forceinline__ real stage_face_own(const SweepArgs<real>& a, const r
         prim_load(a, c + 2 * s, W[3]);
         return plm_flux<real, RS>(a, W, bn_at(a, c), F);
     } else {
-        return ppm_flux_calc<real, RS, KIND == 3>(a, c, s, F);
+        return ppm_flux_calc<real, RS, false>(a, c, s, F);
     }
 }
 // z face k+1/2: predictor between the thread's own cells of planes k (UL) and k+1 (UR),
@@ -93,7 +90,7 @@ __device__ __forceinline__ real stage_face_z(const SweepArgs<real>& a, const rea
         riemann<RS>(uL, uR, (real)a.cs, F, smax);
         return smax;
     } else if constexpr (KIND >= 2) {
-        return ppm_flux_calc<real, RS, KIND == 3>(a, c, s, F);
+        return ppm_flux_calc<real, RS, false>(a, c, s, F);
     } else {
         return flux_corr_calc<real, RS>(a, c, s, F);
     }
@@ -856,8 +853,7 @@ __global__ __launch_bounds__(TX * TY, VS_WAVES) void k_vl_stage(const BoxDesc* _
 }
 
 // kind: 0 predictor, 1 PLM corrector (both FP32; FP64 runs k_vl_near), 2 PPM-primitive
-// corrector, 3 PPM-characteristic corrector (FP32; FP64 runs k_vl_char); shape 2 exists in
-// FP32 only
+// corrector; the PPM-characteristic corrector runs k_vl_char; shape 2 exists in FP32 only
 template <class real, int RS, int KIND>
 void launch_vl_stage_k(hipStream_t st, const BoxDesc* boxes, const TilePlan& plan, const StageArgs<real>& a,
                        int shape) {
@@ -901,7 +897,7 @@ int vl_stage_blocks_per_cu(int kind, int shape) {
             case 0: return vl_near_blocks_per_cu<RS, true>(shape);
             case 1: return vl_near_blocks_per_cu<RS, false>(shape);
             case 2: return vl_stage_blocks_per_cu_k<real, RS, 2>(shape);
-            default: return vl_char_blocks_per_cu<RS>(shape);
+            default: return vl_char_blocks_per_cu<real, RS>(shape);
         }
     } else {
         switch (kind) {
@@ -910,7 +906,7 @@ int vl_stage_blocks_per_cu(int kind, int shape) {
             case 2: return vl_stage_blocks_per_cu_k<real, RS, 2>(shape);
             case 4: return vl_stage_blocks_per_cu_k<real, RS, 4>(shape);
             case 5: return vl_stage_blocks_per_cu_k<real, RS, 5>(shape);
-            default: return vl_stage_blocks_per_cu_k<real, RS, 3>(shape);
+            default: return vl_char_blocks_per_cu<real, RS>(shape);
         }
     }
 }
@@ -924,7 +920,7 @@ void launch_vl_stage(hipStream_t st, const BoxDesc* boxes, const TilePlan& plan,
             case 0: launch_vl_near<RS, true>(st, boxes, plan, a, shape); break;
             case 1: launch_vl_near<RS, false>(st, boxes, plan, a, shape); break;
             case 2: launch_vl_stage_k<real, RS, 2>(st, boxes, plan, a, shape); break;
-            default: launch_vl_char<RS>(st, boxes, plan, a, shape); break;
+            default: launch_vl_char<real, RS>(st, boxes, plan, a, shape); break;
         }
     } else {
         switch (kind) {
@@ -933,7 +929,7 @@ void launch_vl_stage(hipStream_t st, const BoxDesc* boxes, const TilePlan& plan,
             case 2: launch_vl_stage_k<real, RS, 2>(st, boxes, plan, a, shape); break;
             case 4: launch_vl_stage_k<real, RS, 4>(st, boxes, plan, a, shape); break;
             case 5: launch_vl_stage_k<real, RS, 5>(st, boxes, plan, a, shape); break;
-            default: launch_vl_stage_k<real, RS, 3>(st, boxes, plan, a, shape); break;
+            default: launch_vl_char<real, RS>(st, boxes, plan, a, shape); break;
         }
     }
 }
