@@ -24,8 +24,9 @@
 //   G   update of plane k
 // with a barrier after A1, A2 and D.  Scheduling fences keep the phases' working sets apart,
 // and the thread index is marked as rewritten each plane, so that LDS and global addresses
-// are formed where they are used: hoisted out of the march they took 70 registers.  The own
-// column's planes k, k+2 and k+3 are read again from L2 each plane for the same reason.
+// are formed where they are used: hoisted out of the march they took 70 registers.  FP64 reads
+// the own column's planes k, k+2 and k+3 again from L2 each plane for the same reason; FP32 has
+// the registers to carry them and loads plane k+3 only, at the start of the pass.
 // FP64: two workgroups per CU (75 KB of LDS per 16 x 16 tile, 256 registers): the 65 registers
 // that spill cost less than the second workgroup gains (128^3: 1.10 ms per launch, against
 // 1.36 ms with one workgroup and nothing spilled).
@@ -35,7 +36,9 @@
 // FP32 is the same kernel with the fused operations of the per-face form written out
 // (char_edge, ppm_edge, char_solve), so that its results keep their bits: a rounding moved in
 // an edge value turns up as a different limiter branch in single cells.  Per launch at 256^3
-// (HLLD) 4.02 -> 2.76 ms with 16 x 16 tiles; 32 x 16 tiles take 2.97.
+// (HLLD) 4.02 -> 2.76 ms with 16 x 16 tiles, 2.57 with the own column carried.  It is bound by
+// VALU issue (5470 instructions per cell before the carry, the VALU busy in 90 % of the cycles);
+// four waves per SIMD, by lane shifts in place of 8 KB of LDS, spill 99 registers: 3.5 ms.
 #pragma once
 #include "vl_stage_impl.hpp"
 
@@ -408,6 +411,8 @@ __global__ __launch_bounds__(TX * TY, VC_WAVES) void k_vl_char(const BoxDesc* __
     for (int f = 0; f < 4; f++) fz[f] = dxy[f] = dxn[f] = real(0);
     // z march: E and the limited upper state of plane k, and its upper face field
     real Ez_[6], wRz[6], wbz;
+    constexpr bool CARRY = sizeof(real) == 4;
+    real w0z[CARRY ? 6 : 1], Pn[CARRY ? 7 : 1];   // FP32: the own column's planes k and k+2
     {
         const int tx = (int)(t % TX), ty = (int)(t / TX), i = i0 + tx, j = j0 + ty, own = (ty + 2) * PX + tx + 2;
         real W[4][6], u[7];
@@ -431,6 +436,11 @@ __global__ __launch_bounds__(TX * TY, VC_WAVES) void k_vl_char(const BoxDesc* __
         for (int r = 0; r < 6; r++) {
             W[3][r] = u[rslot<2>(r)];
             wRz[r] = real(0);
+            if constexpr (CARRY) w0z[r] = W[1][r];
+        }
+        if constexpr (CARRY) {
+#pragma unroll
+            for (int f = 0; f < 7; f++) Pn[f] = u[f];
         }
         wbz = face_b(2, i, j, ks - 2);
         char_edge(W, wbz, cs, beta, Ez_);
@@ -455,6 +465,8 @@ __global__ __launch_bounds__(TX * TY, VC_WAVES) void k_vl_char(const BoxDesc* __
         const bool pt = inr(p, a.ft_lo, n2 + a.ft_hi);
         // ---- A1
         const real wby = face_b(1, i, j, p), wbz1 = face_b(2, i, j, p);
+        real P3[7];
+        if constexpr (CARRY) load_cons(i, j, k + 3, P3);
         sEf[0][t] = xez;
         sEf[1][t] = yez;
         sV[0][t] = cz;
@@ -494,19 +506,31 @@ __global__ __launch_bounds__(TX * TY, VC_WAVES) void k_vl_char(const BoxDesc* __
         }
         __builtin_amdgcn_sched_barrier(0);
         {   // z: E of plane k+1, its limited states, face k+1/2
-            real W[4][6], E[6], sl[6], sr[6], P0[7], P2[7], P3[7];
-            load_cons(i, j, k, P0);
-            load_cons(i, j, k + 2, P2);
-            load_cons(i, j, k + 3, P3);
-            to_prims(P0);
-            to_prims(P2);
-            to_prims(P3);
+            real W[4][6], E[6], sl[6], sr[6];
+            if constexpr (CARRY) {
+                to_prims(P3);
 #pragma unroll
-            for (int r = 0; r < 6; r++) {
-                W[0][r] = P0[rslot<2>(r)];
-                W[1][r] = sW[rslot<2>(r)][own];
-                W[2][r] = P2[rslot<2>(r)];
-                W[3][r] = P3[rslot<2>(r)];
+                for (int r = 0; r < 6; r++) {
+                    W[0][r] = w0z[r];
+                    W[1][r] = w0z[r] = sW[rslot<2>(r)][own];
+                    W[2][r] = Pn[rslot<2>(r)];
+                    W[3][r] = P3[rslot<2>(r)];
+                }
+            } else {
+                real P0[7], P2[7];
+                load_cons(i, j, k, P0);
+                load_cons(i, j, k + 2, P2);
+                load_cons(i, j, k + 3, P3);
+                to_prims(P0);
+                to_prims(P2);
+                to_prims(P3);
+#pragma unroll
+                for (int r = 0; r < 6; r++) {
+                    W[0][r] = P0[rslot<2>(r)];
+                    W[1][r] = sW[rslot<2>(r)][own];
+                    W[2][r] = P2[rslot<2>(r)];
+                    W[3][r] = P3[rslot<2>(r)];
+                }
             }
             char_edge(W, wbz1, cs, beta, E);
 #pragma unroll
@@ -616,7 +640,7 @@ __global__ __launch_bounds__(TX * TY, VC_WAVES) void k_vl_char(const BoxDesc* __
         const bool ccb = lb(LB_CCB) && k >= a.u_lo + sh;
         real w2[7], g[7];
         int rx = 0, ry = 0;
-        load_cons(i, j, k + 2, w2);
+        if constexpr (!CARRY) load_cons(i, j, k + 2, w2);
         if (t < NR) {
             ring_xy(rx, ry);
             load_cons(i0 + rx, j0 + ry, k + 2, g);
@@ -665,9 +689,17 @@ __global__ __launch_bounds__(TX * TY, VC_WAVES) void k_vl_char(const BoxDesc* __
                 sEc[q0][0][t] = (0.25 * (y0 + y1 + z0 + z1) + 0.25 * ((a14 - a34) + (b14 - b34)));
             }
         }
-        to_prims(w2);
+        if constexpr (CARRY) {
 #pragma unroll
-        for (int f = 0; f < 7; f++) sW[f][own] = w2[f];
+            for (int f = 0; f < 7; f++) {
+                sW[f][own] = Pn[f];
+                Pn[f] = P3[f];
+            }
+        } else {
+            to_prims(w2);
+#pragma unroll
+            for (int f = 0; f < 7; f++) sW[f][own] = w2[f];
+        }
         if (t < NR) {
             to_prims(g);
 #pragma unroll
