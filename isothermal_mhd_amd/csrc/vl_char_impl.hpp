@@ -36,7 +36,7 @@
 // FP32 is the same kernel with the fused operations of the per-face form written out
 // (char_edge, ppm_edge, char_solve), so that its results keep their bits: a rounding moved in
 // an edge value turns up as a different limiter branch in single cells.  Per launch at 256^3
-// (HLLD) 4.02 -> 2.76 ms with 16 x 16 tiles, 2.57 with the own column carried.  It is bound by
+// (HLLD) 4.02 -> 2.76 ms with 16 x 16 tiles, 2.61 with the own column carried.  It is bound by
 // VALU issue (5470 instructions per cell before the carry, the VALU busy in 90 % of the cycles);
 // four waves per SIMD, by lane shifts in place of 8 KB of LDS, spill 99 registers: 3.5 ms.
 #pragma once
