@@ -129,13 +129,15 @@ __global__ __launch_bounds__(256) void k_max_speed(const BoxDesc* __restrict__ b
 }
 
 // dt = COUR dx / max(cmax, smax + delv_max), then MIN(t_end - t, dt) (driver.f90:432-448, 475)
-__global__ void k_new_dt(int nbox, const BoxDesc* __restrict__ boxes, const unsigned long long* cmax,
+// One wavefront per box: its lanes read the slots of the maxima (one thread that walked 3 x 64
+// lines of memory took 9 us).
+__global__ __launch_bounds__(64) void k_new_dt(const BoxDesc* __restrict__ boxes, const unsigned long long* cmax,
                          const unsigned long long* smax, const unsigned long long* dvmax, const double* cour,
                          double t_end, double* t, double* dt, double* dt_prev, int advance_time) {
-    int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nbox) return;
+    const int b = blockIdx.x;
     double cm = striped_max(cmax, b);
     double sm = striped_max(smax, b) + striped_max(dvmax, b);   // smax + delv_max (vanleer_mod.f90:3323)
+    if (threadIdx.x != 0) return;
     double c = fmax(cm, sm);
     if (advance_time) t[b] = t[b] + dt[b];
     dt_prev[b] = dt[b];
@@ -147,6 +149,14 @@ __global__ void k_new_dt(int nbox, const BoxDesc* __restrict__ boxes, const unsi
 __global__ void k_reset_u64(unsigned long long* p, int n) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = 0ull;
+}
+// Up to three arrays of n values each (b, c may be null): a step's maxima in one launch
+__global__ void k_reset_maxima(unsigned long long* a, unsigned long long* b, unsigned long long* c, int n) {
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    a[i] = 0ull;
+    if (b != nullptr) b[i] = 0ull;
+    if (c != nullptr) c[i] = 0ull;
 }
 
 // ---------------------------------------------------------------------------------
@@ -683,8 +693,11 @@ void launch_pass_update(const Launch& L, const PassUpdArgs<real>& a) {
 void launch_new_dt(hipStream_t st, int nbox, const BoxDesc* boxes, const unsigned long long* cmax,
                    const unsigned long long* smax, const unsigned long long* dvmax, const double* cour, double t_end,
                    double* t, double* dt, double* dt_prev, int advance_time) {
-    hipLaunchKernelGGL(k_new_dt, dim3((nbox + 63) / 64), dim3(64), 0, st, nbox, boxes, cmax, smax, dvmax, cour, t_end,
+    hipLaunchKernelGGL(k_new_dt, dim3((unsigned)nbox), dim3(64), 0, st, boxes, cmax, smax, dvmax, cour, t_end,
                        t, dt, dt_prev, advance_time);
+}
+void launch_reset_maxima(hipStream_t st, unsigned long long* a, unsigned long long* b, unsigned long long* c, int n) {
+    hipLaunchKernelGGL(k_reset_maxima, dim3((n + 255) / 256), dim3(256), 0, st, a, b, c, n);
 }
 void launch_reset_u64(hipStream_t st, unsigned long long* p, int n) {
     hipLaunchKernelGGL(k_reset_u64, dim3((n + 255) / 256), dim3(256), 0, st, p, n);

@@ -731,10 +731,10 @@ void protection_fix(imhd_ctx* c, int src, bool corrector) {
     launch_prot_fix(mk(c, c->pl_ghost), a);
 }
 
+// (clear_cmax: native steps, whose CFL speed follows; delv_max = 0 as in vanleer_mod.f90:301)
 template <class real>
-void vl_step(imhd_ctx* c, bool fuse_cmax = false, bool with_passive = false) {
-    launch_reset_u64(c->st, c->smax, (int)stripe_slots(c->nbox));
-    launch_reset_u64(c->st, c->dvmax, (int)stripe_slots(c->nbox));   // delv_max = 0 (vanleer_mod.f90:301)
+void vl_step(imhd_ctx* c, bool fuse_cmax = false, bool with_passive = false, bool clear_cmax = false) {
+    launch_reset_maxima(c->st, c->smax, c->dvmax, clear_cmax ? c->cmax : nullptr, (int)stripe_slots(c->nbox));
     const int s0 = c->cur, s1 = 1 - c->cur;
     if (with_passive) {
         vl_stage<real>(c, s0, s0, 2, false, false, "stage_pred", true);
@@ -856,8 +856,9 @@ void tvd_corner(imhd_ctx* c, int s0, bool corr) {
 // One tvd_solve_3d.  Buffers: t^n in state/face set s0; the CT half-step faces, the CTU
 // half states and finally the new state in set s1.
 template <class real>
-void tvd_step(imhd_ctx* c) {
-    launch_reset_u64(c->st, c->smax, (int)stripe_slots(c->nbox));  // no smax in the TVD module
+void tvd_step(imhd_ctx* c, bool clear_cmax = false) {
+    // no smax in the TVD module
+    launch_reset_maxima(c->st, c->smax, clear_cmax ? c->cmax : nullptr, nullptr, (int)stripe_slots(c->nbox));
     const int s0 = c->cur, s1 = 1 - c->cur;
     for (int d = 0; d < 3; d++) tvd_sweep<real>(c, s0, s0, false, d);
     tvd_corner<real>(c, s0, false);
@@ -943,9 +944,9 @@ void tvd_step(imhd_ctx* c) {
 }
 
 template <class real>
-void tvd_max_speed_launch(imhd_ctx* c) {
+void tvd_max_speed_launch(imhd_ctx* c, bool cleared = false) {
     ProfScope ps(c, "max_speed_tvd", c->pl_tcfl.active);
-    launch_reset_u64(c->st, c->cmax, (int)stripe_slots(c->nbox));
+    if (!cleared) launch_reset_u64(c->st, c->cmax, (int)stripe_slots(c->nbox));
     QPtrs<real> q{};
     for (int f = 0; f < 7; f++) q.q[f] = R<real>(c->q[c->cur][f]);
     launch_tvd_max_speed<real>(mk(c, c->pl_tcfl), q, c->cfg.cs, c->cmax);
@@ -1145,18 +1146,17 @@ void native_step(imhd_ctx* c, double t_end) {
     const int qold = c->cur;
     c->trim = c->trim_ok && c->ghost_images;
     if (is_tvd(c)) {  // driver.f90:35-160 order: solve, passive, new dt, then ghost fill
-        tvd_step<real>(c);
+        tvd_step<real>(c, true);
         if (c->ou_on) ou_step<real>(c, false);
         if (c->cfg.npass > 0) passive_fused<real>(c, qold);
-        tvd_max_speed_launch<real>(c);
+        tvd_max_speed_launch<real>(c, true);
         fill_ghosts<real>(c);
         c->trim = false;
         launch_new_dt(c->st, c->nbox, c->db, c->cmax, c->smax, c->dvmax, c->cour, t_end, c->t, c->dt, c->dtprev, 1);
         return;
     }
-    launch_reset_u64(c->st, c->cmax, (int)stripe_slots(c->nbox));
     const bool inl = c->pvel[0] != nullptr && !c->ou_on;
-    vl_step<real>(c, !c->ou_on, inl);
+    vl_step<real>(c, !c->ou_on, inl, true);
     if (c->ou_on) ou_step<real>(c, true);   // the CFL speed is taken after the kick
     if (c->cfg.npass > 0 && !inl) passive_fused<real>(c, qold);
     fill_ghosts<real>(c);

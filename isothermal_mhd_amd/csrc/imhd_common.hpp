@@ -275,10 +275,12 @@ __device__ __forceinline__ void atomic_max_nonneg(unsigned long long* base, int 
         if (bits > __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(a, bits);
     }
 }
+// Maximum over a box's slots, one per lane of a wavefront (all lanes active)
 __device__ __forceinline__ double striped_max(const unsigned long long* base, int box) {
-    unsigned long long m = 0;
-    for (int s = 0; s < NSTRIPE; s++) {
-        unsigned long long v = base[((size_t)box * NSTRIPE + s) * STRIPE_STRIDE];
+    static_assert(NSTRIPE == 64, "one slot per lane");
+    unsigned long long m = base[((size_t)box * NSTRIPE + (threadIdx.x & 63)) * STRIPE_STRIDE];
+    for (int o = 32; o > 0; o >>= 1) {
+        const unsigned long long v = __shfl_xor(m, o, 64);
         m = v > m ? v : m;
     }
     return __longlong_as_double((long long)m);
