@@ -17,16 +17,20 @@ __device__ __forceinline__ int bc_map(int i, int n, int bc) {
     return i < 1 ? 1 : n;                         // open: copy the edge cell
 }
 
-// Copies cell s to cell d in the fill's first n fields of type real and in its FP64 ones.
+// Copies cell s to cell d in the fill's first n fields of type real and in its FP64 ones, if
+// it has any.
 // Eight fields' loads are issued before their stores, which may alias a later load.  The x
 // sides bound it (12 cells of every row's lines): 158 B per cell moved of 104 needed, 3.5 TB/s
 // (FP32 256^3, 0.11 ms).  The passives come along instead of in a launch of their own, which
 // took 7 us on the smallest boxes.
 template <class real>
 __device__ __forceinline__ void copy_fields(const GhostArgs<real>& a, int n, long long d, long long s) {
+    const bool faces = a.d[0] != nullptr;
     double w[3];
+    if (faces) {
 #pragma unroll
-    for (int u = 0; u < 3; u++) w[u] = a.d[u][s];
+        for (int u = 0; u < 3; u++) w[u] = a.d[u][s];
+    }
     for (int f0 = 0; f0 < n; f0 += 8) {
         real v[8];
 #pragma unroll
@@ -36,8 +40,10 @@ __device__ __forceinline__ void copy_fields(const GhostArgs<real>& a, int n, lon
         for (int u = 0; u < 8; u++)
             if (f0 + u < n) a.r[f0 + u][d] = v[u];
     }
+    if (faces) {
 #pragma unroll
-    for (int u = 0; u < 3; u++) a.d[u][d] = w[u];
+        for (int u = 0; u < 3; u++) a.d[u][d] = w[u];
+    }
 }
 
 // It enumerates only the ghost band of depth w around the interior: the plan gives each box

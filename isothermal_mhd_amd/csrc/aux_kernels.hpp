@@ -16,7 +16,7 @@ hipError_t diag_static_scratch(double** out);
 template <class real>
 struct GhostArgs {
     real* r[7 + MAXPASS];
-    double* d[3];
+    double* d[3];         // all three or none
     int nreal, depth;     // fields r[0 .. nreal) and d, to this depth
     int nreal2, depth2;   // and r[nreal .. nreal2), the passives, to depth2 <= depth
 };
