@@ -106,8 +106,8 @@ struct imhd_ctx {
     bool fft_have_plan = false;
     int fft_n = 0;
     unsigned long long fft_bytes = 0;   // plan work area and buffers (in dev_bytes too)
-    // n^2 (n/2+1) complex each: packed components (n^3 floats) and transforms.  A density
-    // spectrum uses fft_in and fft_out[0], everything else all four
+    // n^2 (n/2+1) complex each: packed components (n^3 floats) and transforms.  A spectrum
+    // needs fft_in and fft_out[0], the mode spectra all four
     void* fft_in = nullptr;
     void* fft_out[3] = {};
     void* fft_acc = nullptr;        // (n/2)^3 floats (octant power)
@@ -2050,16 +2050,11 @@ static int spectrum_t(imhd_ctx* c, int bx, int which, double* k_out, double* pk_
     const int ncomp = which == SPEC_DENSITY ? 1 : 3;
     int rc = fft_setup(c, n, 1);
     if (rc) return rc;
-    // three components are packed in one pass where there is ample room for them: in fft_in and
-    // the last two transform buffers (at most a quarter of the free memory, if they have yet
-    // to be made), the transforms one after the other in the first
-    bool together = ncomp == 3 && !getenv("IMHD_TEST_SPEC_SINGLE");   // tests: as if there were no room
-    if (together && !(c->fft_out[1] && c->fft_out[2])) {
-        size_t room = 0, total = 0;
-        together = hipMemGetInfo(&room, &total) == hipSuccess &&
-                   2 * ((size_t)n * n * (h + 1) * 8) <= room / 4 && fft_setup(c, n, 3) == IMHD_OK;
-        if (!together) (void)hipGetLastError();
-    }
+    // once the mode spectra have made their buffers, three components are packed in one pass:
+    // in fft_in and the last two transform buffers, the transforms one after the other in the
+    // first.  Buffers are not made for it: a context keeps them, and the next larger
+    // allocation may need the room more than a spectrum needs one launch instead of three
+    const bool together = ncomp == 3 && c->fft_out[1] && c->fft_out[2];
     struct Raw { double* p; };   // the cached buffers, in the form the launch calls take
     const Raw fout{(double*)c->fft_out[0]}, acc{(double*)c->fft_acc}, pk{(double*)c->fft_bins};
     const hipfftHandle plan = c->fft_plan;
