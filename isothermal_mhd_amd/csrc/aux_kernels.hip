@@ -17,20 +17,16 @@ __device__ __forceinline__ int bc_map(int i, int n, int bc) {
     return i < 1 ? 1 : n;                         // open: copy the edge cell
 }
 
-// Copies cell s to cell d in the fill's first n fields of type real and in its FP64 ones, if
-// it has any.
+// Copies cell s to cell d in the fill's first n fields of type real and in its FP64 ones.
 // Eight fields' loads are issued before their stores, which may alias a later load.  The x
 // sides bound it (12 cells of every row's lines): 158 B per cell moved of 104 needed, 3.5 TB/s
 // (FP32 256^3, 0.11 ms).  The passives come along instead of in a launch of their own, which
 // took 7 us on the smallest boxes.
 template <class real>
 __device__ __forceinline__ void copy_fields(const GhostArgs<real>& a, int n, long long d, long long s) {
-    const bool faces = a.d[0] != nullptr;
     double w[3];
-    if (faces) {
 #pragma unroll
-        for (int u = 0; u < 3; u++) w[u] = a.d[u][s];
-    }
+    for (int u = 0; u < 3; u++) w[u] = a.d[u][s];
     for (int f0 = 0; f0 < n; f0 += 8) {
         real v[8];
 #pragma unroll
@@ -40,27 +36,17 @@ __device__ __forceinline__ void copy_fields(const GhostArgs<real>& a, int n, lon
         for (int u = 0; u < 8; u++)
             if (f0 + u < n) a.r[f0 + u][d] = v[u];
     }
-    if (faces) {
 #pragma unroll
-        for (int u = 0; u < 3; u++) a.d[u][d] = w[u];
-    }
+    for (int u = 0; u < 3; u++) a.d[u][d] = w[u];
 }
 
-// It enumerates only the ghost band of depth w around the interior: the plan gives each box
-// r[0] = number of band cells; the linear index is decoded as z-slabs, then
-// y-slabs (interior k), then x-slabs (interior j, k).
-template <class real>
-__global__ __launch_bounds__(256) void k_fill_ghost_band(const BoxDesc* __restrict__ boxes, Plan plan, GhostArgs<real> a) {
-    int b, g, dum1, dum2;
-    if (!plan_item(plan, b, g, dum1, dum2)) return;
-    const BoxDesc& B = boxes[b];
-    const int w = a.depth;
+// Cell t of the ghost band of depth w around a box's interior: z-slabs, then y-slabs (interior
+// k), then x-slabs (interior j, k).
+__device__ __forceinline__ void band_cell(const BoxDesc& B, unsigned t, int w, int& i, int& j, int& k) {
     // 32-bit decoding: the plan holds a band's number of cells in an int
     const unsigned W = 2u * (unsigned)w, E0 = (unsigned)B.n[0] + W, E1 = (unsigned)B.n[1] + W;
     const unsigned nA = E0 * E1 * W, nB = E0 * W * (unsigned)B.n[2];
-    unsigned t = (unsigned)g;
     auto side = [&](unsigned s, int n) { return (int)s < w ? 1 - w + (int)s : n + 1 + (int)s - w; };
-    int i, j, k;
     if (t < nA) {
         const unsigned row = t / E0, kk = row / E1;
         k = side(kk, B.n[2]);
@@ -79,11 +65,38 @@ __global__ __launch_bounds__(256) void k_fill_ghost_band(const BoxDesc* __restri
         j = 1 + (int)(u - kk * (unsigned)B.n[1]);
         k = 1 + (int)kk;
     }
-    const int si = bc_map(i, B.n[0], B.bc), sj = bc_map(j, B.n[1], B.bc), sk = bc_map(k, B.n[2], B.bc);
-    const long long d = cell_index(B, i, j, k), s = cell_index(B, si, sj, sk);
-    const bool inner = i >= 1 - a.depth2 && j >= 1 - a.depth2 && k >= 1 - a.depth2 && i <= B.n[0] + a.depth2 &&
-                       j <= B.n[1] + a.depth2 && k <= B.n[2] + a.depth2;
-    copy_fields(a, inner ? a.nreal2 : a.nreal, d, s);
+}
+__device__ __forceinline__ bool within(const BoxDesc& B, int i, int j, int k, int w) {
+    return i >= 1 - w && j >= 1 - w && k >= 1 - w && i <= B.n[0] + w && j <= B.n[1] + w && k <= B.n[2] + w;
+}
+__device__ __forceinline__ long long ghost_source(const BoxDesc& B, int i, int j, int k) {
+    return cell_index(B, bc_map(i, B.n[0], B.bc), bc_map(j, B.n[1], B.bc), bc_map(k, B.n[2], B.bc));
+}
+
+// The plan gives each box r[0] = number of cells of its band of depth a.depth
+template <class real>
+__global__ __launch_bounds__(256) void k_fill_ghost_band(const BoxDesc* __restrict__ boxes, Plan plan, GhostArgs<real> a) {
+    int b, g, dum1, dum2, i, j, k;
+    if (!plan_item(plan, b, g, dum1, dum2)) return;
+    const BoxDesc& B = boxes[b];
+    band_cell(B, (unsigned)g, a.depth, i, j, k);
+    const long long d = cell_index(B, i, j, k), s = ghost_source(B, i, j, k);
+    copy_fields(a, within(B, i, j, k, a.depth2) ? a.nreal2 : a.nreal, d, s);
+}
+
+// The same for the compensation terms of the FP32 state, to depth a.depth2 only (same plan)
+__global__ __launch_bounds__(256) void k_fill_comp_ghosts(const BoxDesc* __restrict__ boxes, Plan plan, CompGhostArgs a) {
+    int b, g, dum1, dum2, i, j, k;
+    if (!plan_item(plan, b, g, dum1, dum2)) return;
+    const BoxDesc& B = boxes[b];
+    band_cell(B, (unsigned)g, a.depth, i, j, k);
+    if (!within(B, i, j, k, a.depth2)) return;
+    const long long d = cell_index(B, i, j, k), s = ghost_source(B, i, j, k);
+    float v[4];
+#pragma unroll
+    for (int f = 0; f < 4; f++) v[f] = a.comp[f][s];
+#pragma unroll
+    for (int f = 0; f < 4; f++) a.comp[f][d] = v[f];
 }
 
 // Cells outside [lo, n + hi_off] (any axis) take their t^n values: the state the
@@ -632,6 +645,9 @@ template void launch_prot_fix<float>(const Launch&, const ProtArgs<float>&);
 template <class real>
 void launch_fill_ghost_band(const Launch& L, const GhostArgs<real>& a) {
     if (L.plan.total > 0) L256((k_fill_ghost_band<real>), L.boxes, L.plan, a);
+}
+void launch_fill_comp_ghosts(const Launch& L, const CompGhostArgs& a) {
+    if (L.plan.total > 0) L256(k_fill_comp_ghosts, L.boxes, L.plan, a);
 }
 template <class real>
 void launch_restore_shell(const Launch& L, const ShellArgs<real>& a) {

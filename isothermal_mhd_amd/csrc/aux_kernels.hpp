@@ -16,9 +16,14 @@ hipError_t diag_static_scratch(double** out);
 template <class real>
 struct GhostArgs {
     real* r[7 + MAXPASS];
-    double* d[3];         // all three or none
+    double* d[3];
     int nreal, depth;     // fields r[0 .. nreal) and d, to this depth
     int nreal2, depth2;   // and r[nreal .. nreal2), the passives, to depth2 <= depth
+};
+
+struct CompGhostArgs {
+    float* comp[4];
+    int depth, depth2;    // of the plan's band, of the cells filled
 };
 
 template <class real>
@@ -122,6 +127,7 @@ template <class real> void launch_prot_fix(const Launch& L, const ProtArgs<real>
 
 template <class real> void launch_restore_shell(const Launch& L, const ShellArgs<real>& a);
 template <class real> void launch_fill_ghost_band(const Launch& L, const GhostArgs<real>& a);
+void launch_fill_comp_ghosts(const Launch& L, const CompGhostArgs& a);
 template <class real> void launch_pass_stage(const Launch& L, const PassStageArgs<real>& a);
 template <class real> void launch_max_speed(const Launch& L, const QPtrs<real>& q, double cs, unsigned long long* cmax);
 template <class real> void launch_diag(hipStream_t st, const BoxDesc* boxes, int nbox, const DiagArgs<real>& a);

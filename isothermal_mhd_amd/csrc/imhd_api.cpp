@@ -1062,12 +1062,11 @@ void fill_comp_ghosts(imhd_ctx* c) {
     if (!c->comp_behind) return;
     c->comp_behind = false;
     if (c->comp[0] == nullptr || is_tvd(c)) return;
-    GhostArgs<float> g{};
-    for (int f = 0; f < 4; f++) g.r[f] = R<float>(c->comp[f]);
+    CompGhostArgs g{};
+    for (int f = 0; f < 4; f++) g.comp[f] = R<float>(c->comp[f]);
     g.depth = c->hb[0].nb;
-    g.nreal2 = 4;
     g.depth2 = c->hb[0].nb - 4 - (c->cfg.recon == IMHD_PLM_PRIM ? 0 : 1);
-    launch_fill_ghost_band<float>(mk(c, c->pl_gband), g);
+    launch_fill_comp_ghosts(mk(c, c->pl_gband), g);
 }
 
 template <class real>
