@@ -126,16 +126,14 @@ def run_c2(n, steps, warmup, cour, recon="plm"):
     r32 = run_path(state0, n, 32, steps, warmup, cour, recon)
     r64 = run_path(state0, n, 64, steps, warmup, cour, recon)
     v32, v64 = n ** 3 * steps / r32["sec"] / 1e6, n ** 3 * steps / r64["sec"] / 1e6
-    roof = roofline(r32["prof"], 4, n ** 3, 1, r32["sec"] / steps * 1e3, f"c2_{n}")
-    if recon == "ppm_char" and roof["kernel"].startswith("stage_corr"):
-        roof["symbol"] = "k_vl_char"
     return {"value": v32, "unit": "Mcell-updates/s", "steps": steps, "dtype": "f32",
             "ms_per_step": r32["sec"] / steps * 1e3, "graph_value": n ** 3 * steps / r32["graph_sec"] / 1e6,
             "fp64": {"value": v64, "ms_per_step": r64["sec"] / steps * 1e3,
                      "graph_value": n ** 3 * steps / r64["graph_sec"] / 1e6, "max_divb": r64["diag"]["divb_max"]},
             "fp32_over_fp64": v32 / v64, "max_divb": r32["diag"]["divb_max"], "autotune": r32["autotune"],
             "l1_fp32_vs_fp64": l1_errors(r32["state"], r64["state"]),
-            "roofline": roof, "kernels_fp32_ms": {k: round(v[0] / v[1], 5) for k, v in r32["prof"].items()},
+            "roofline": roofline(r32["prof"], 4, n ** 3, 1, r32["sec"] / steps * 1e3, f"c2_{n}", recon),
+            "kernels_fp32_ms": {k: round(v[0] / v[1], 5) for k, v in r32["prof"].items()},
             "workload": f"{n}^3 periodic, VL2+CT, HLLD, "
                         + ("primitive PLM" if recon == "plm" else "characteristic PPM (the reference's default)")
                         + ", 1 passive scalar; rho=1, B0=(0,0,1), solenoidal k^-2 velocity 1<=|k|<=8 at rms Mach 2 "
@@ -266,12 +264,13 @@ def b_alg(esz, npass):
     return 2 * (4 * esz + 3 * 8 + npass * esz)
 
 
-def roofline(prof, esz, cells, npass, step_ms, tag):
+def roofline(prof, esz, cells, npass, step_ms, tag, recon="plm"):
     """Roofline of the dominant kernel family (largest total event time): the algorithmic
     bytes of one cell-update (b_alg) times the cells one launch updates, over the average
     launch time, against MI355X's HBM peak; beside it the kernel's own compulsory bytes per
     work item (bytes_per_item), the whole step at b_alg, and the measured HBM traffic of the
-    same workload (profiles/pmc_traffic.json, when it was measured on `tag`)."""
+    same workload (profiles/pmc_traffic.json, when it was measured on `tag` with as many work
+    items per launch)."""
     fam = {}
     for name, (ms, nl, items) in prof.items():
         key = name[:-2] if name[-2:] in ("_x", "_y", "_z") else name
@@ -284,7 +283,7 @@ def roofline(prof, esz, cells, npass, step_ms, tag):
     avg_ms = ms / nl
     ba = b_alg(esz, npass)
     ach = ba * cells / (avg_ms * 1e-3) / 1e9
-    out = {"bound": "hbm", "kernel": key, "symbol": FAMILY_SYMBOL.get(key), "launches": nl,
+    out = {"bound": "hbm", "kernel": key, "symbol": kernel_symbol(key, esz, recon), "launches": nl,
            "avg_launch_ms": avg_ms, "cell_updates_per_launch": cells, "bytes_per_cell_update": ba,
            "achieved": ach, "peak": PEAK_HBM_GBS, "unit": "GB/s", "frac": ach / PEAK_HBM_GBS, "traffic": None,
            "whole_step": {"achieved": ba * cells / (step_ms * 1e-3) / 1e9,
@@ -298,7 +297,7 @@ def roofline(prof, esz, cells, npass, step_ms, tag):
     if os.path.exists(pmc):
         with open(pmc) as f:
             tr = json.load(f)
-        if tr.get("_workload") == tag and key in tr:
+        if tr.get("_workload") == tag and key in tr and tr.get("_items", {}).get(key) == items // nl:
             out["traffic"] = tr[key]
             out["measured"] = {"achieved": tr[key] / (avg_ms * 1e-3) / 1e9,
                                "frac": tr[key] / (avg_ms * 1e-3) / 1e9 / PEAK_HBM_GBS,
@@ -309,21 +308,31 @@ def roofline(prof, esz, cells, npass, step_ms, tag):
     if esz == 4 and os.path.exists(sq):
         with open(sq) as f:
             vq = json.load(f)
-        if vq.get("_workload") == tag and key in vq:
+        if vq.get("_workload") == tag and key in vq and vq.get("_items", {}).get(key) == items // nl:
             a3 = vq[key]["valu_wave_instr"] / (avg_ms * 1e-3) / 1e9
             out["valu_issue"] = {"achieved": a3, "peak": VALU_PEAK_GWI, "unit": "G wave-instr/s",
                                  "frac": a3 / VALU_PEAK_GWI, "wave_instr_per_launch": vq[key]["valu_wave_instr"]}
     return out
 
 
-# family (bench profiler name) -> kernel symbol it launches (fused three-direction sweeps,
-# z-marching column updates)
-FAMILY_SYMBOL = {"stage_pred": "k_vl_stage", "stage_corr_cfl": "k_vl_stage",
-                 "flux_pred": "k_flux3", "flux_corr": "k_flux3", "corner_pred": "k_corner",
-                 "corner_corr": "k_corner", "update_pred": "k_update_z", "update_corr_cfl": "k_update_z",
-                 "pass_stage_pred": "k_pass_stage_z", "pass_stage_corr": "k_pass_stage_z",
-                 "fill_ghosts": "k_fill_ghost_band", "fill_ghosts_pass": "k_fill_ghost_band",
-                 "stage_corr": "k_vl_stage", "ou_forcing": "k_ou_kick"}
+# families (profiler names) whose kernel does not depend on precision or reconstruction
+FAMILY_SYMBOL = {"flux_pred": "k_flux3", "flux_corr": "k_flux3", "corner_pred": "k_corner_z",
+                 "corner_corr": "k_corner_z", "update_pred": "k_update_z", "update_corr": "k_update_z",
+                 "update_corr_cfl": "k_update_z", "pass_stage_pred": "k_pass_stage_z",
+                 "pass_stage_corr": "k_pass_stage_z", "fill_ghosts": "k_fill_ghost_band", "ou_forcing": "k_ou_kick"}
+
+
+def kernel_symbol(family, esz, recon="plm"):
+    """The kernel that launches of a family run, None for a family that is not counted.  The
+    fused VL stages: the characteristic PPM corrector has its own kernel; the predictor and
+    the PLM corrector have one in FP64; the others run k_vl_stage."""
+    if family in ("stage_pred", "stage_corr", "stage_corr_cfl"):
+        if family != "stage_pred" and recon == "ppm_char":
+            return "k_vl_char"
+        if esz == 8 and (family == "stage_pred" or recon == "plm"):
+            return "k_vl_near"
+        return "k_vl_stage"
+    return FAMILY_SYMBOL.get(family)
 
 
 # kernel dispatches of a family's symbol per launch of the family, where not one
@@ -348,8 +357,9 @@ def pmc_run(n=1024, steps=3, n_cal=256, map_path=None):
     fam = {}
     for name, (ms, nl, items) in prof.items():
         key = name[:-2] if name[-2:] in ("_x", "_y", "_z") else name
-        if key in FAMILY_SYMBOL:
-            fam[key] = {"symbol": FAMILY_SYMBOL[key], "order": len(fam), "launches": nl,
+        symbol = kernel_symbol(key, 4)
+        if symbol:
+            fam[key] = {"symbol": symbol, "order": len(fam), "launches": nl,
                         "per_launch": FAMILY_DISPATCHES.get(key, 1), "items": items // nl}
     q, bf, qp = ics.config_c2(n=n_cal)
     C = VanLeerSolver((n_cal,) * 3, npass=1, riemann="hlld", bc="periodic", precision=32)
@@ -431,7 +441,7 @@ def pmc_summarize(fetch_dir, write_dir, map_path=None):
         meas = dv[-1] * 1024.0 / f_fac
         check = {"kernel": ck["symbol"], "bytes_read_known": ck["bytes_read"], "bytes_read_calibrated": meas,
                  "ratio": meas / ck["bytes_read"]}
-    out = {"_workload": mp["workload"],
+    out = {"_workload": mp["workload"], "_items": {k: v["items"] for k, v in mp["families"].items()},
            "_calibration": {"kernel": sym, "bytes_read": cp["bytes_read"], "bytes_written": cp["bytes_written"],
                             "FETCH_SIZE_KiB": cf, "WRITE_SIZE_KiB": cw, "fetch_factor": f_fac, "write_factor": w_fac,
                             "check": check}}
@@ -467,7 +477,8 @@ def sq_summarize(sq_dir, map_path=None):
         mp = json.load(f)
     per = {c: _family_values(_read_counter(sq_dir, c), mp)
            for c in ("SQ_INSTS_VALU", "SQ_ACTIVE_INST_VALU", "SQ_WAVE_CYCLES", "SQ_WAVES")}
-    out = {"_workload": mp["workload"], "_peak_G_wave_instr_per_s": VALU_PEAK_GWI}
+    out = {"_workload": mp["workload"], "_items": {k: v["items"] for k, v in mp["families"].items()},
+           "_peak_G_wave_instr_per_s": VALU_PEAK_GWI}
     lines = ["| family | kernel | VALU wave-instr / launch | VALU instr / wave | active VALU / wave-cycles |",
              "|---|---|---|---|---|"]
     for key, v in sorted(mp["families"].items(), key=lambda kv: kv[1]["order"]):
