@@ -140,7 +140,7 @@ struct imhd_ctx {
     // plans
     PlanDev pl_pflux[3], pl_pcorner, pl_pupd, pl_cflux[3], pl_ccorner, pl_cupd;
     PlanDev pl_gband;
-    PlanDev pl_ghost, pl_pghost, pl_int, pl_vel, pl_ppflux[3], pl_ppupd, pl_pcflux[3], pl_pfupd;
+    PlanDev pl_ghost, pl_int, pl_vel, pl_ppflux[3], pl_ppupd, pl_pcflux[3], pl_pfupd;
     PlanDev pl_pstage[2];   // fused passive stages (column plans when zseg > 0)
     PlanDev pl_teig_p[2][3], pl_tflux_p[3], pl_teig_c[2][3], pl_tflux_c[3];
     PlanDev pl_tsweep_p[2][3], pl_tsweep_c[2][3];   // fused Roe-TVD sweeps
@@ -287,8 +287,6 @@ int build_plan(imhd_ctx* c, PlanDev& p, int which, int dir, int seg = 0, bool tr
                     lo = 5 - nb + e; hi = n + nb - 4 - e; break;
                 case 6:  // whole padded box
                     lo = 1 - nb; hi = n + nb; break;
-                case 7:  // passive ghost band
-                    lo = -2; hi = n + 3; break;
                 case 8:  // interior
                     lo = 1; hi = n; break;
                 case 9:  // copy_velocity (passive_mod.f90:212-214)
@@ -302,10 +300,6 @@ int build_plan(imhd_ctx* c, PlanDev& p, int which, int dir, int seg = 0, bool tr
                 case 13:  // passive final update (offset 2)
                     lo = 1; hi = n; break;
                 // K98 TVD integrator (isotvd_mod.f90); offset 0 predictor, 2 corrector
-                case 25:  // union of the three predictor flux ranges (fused sweeps)
-                    lo = 1 - nb; hi = n + nb; break;
-                case 26:  // union of the three corrector flux ranges (their transverse range)
-                    lo = 3 - nb; hi = n + nb - 2; break;
                 case 16:  // predictor Roe average / HLLE faces: pencil cells [1-nb, n+nb]
                     lo = 1 - nb; hi = normal ? n + nb - 1 : n + nb; break;
                 case 17:  // predictor TVD fluxes and face EMFs (isotvd_mod.f90:2413, 446)
@@ -2339,7 +2333,6 @@ int imhd_create_ensemble(const imhd_config* cfg, int nbox, imhd_ctx** out) {
     if ((rc = build_plan(c, c->pl_cupd, 5, -1, c->zseg))) return rc;
     if ((rc = build_plan(c, c->pl_ghost, 6, -1))) return rc;
     if ((rc = build_plan(c, c->pl_gband, 14, -1))) return rc;
-    if ((rc = build_plan(c, c->pl_pghost, 7, -1))) return rc;
     if ((rc = build_plan(c, c->pl_int, 8, -1))) return rc;
     if ((rc = build_plan(c, c->pl_vel, 9, -1))) return rc;
     if ((rc = build_plan(c, c->pl_ppupd, 11, -1))) return rc;

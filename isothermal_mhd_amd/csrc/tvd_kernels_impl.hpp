@@ -418,7 +418,8 @@ __global__ __launch_bounds__(256) void k_tvd_sweep_x(const BoxDesc* __restrict__
 // y / z sweep: threads along x (coalesced), each marching a segment of pb.seg flux faces
 // along the sweep axis with a three-face window of g~_k in registers.  Items enumerate
 // (x, transverse index, segment), x fastest.
-// FP32 only; FP64 runs k_tvd_sweep_x64 and k_tvd_sweep_yz64 below.
+// This and the x sweep: FP32 only (templates, so that the FP64 file does not compile them);
+// FP64 runs k_tvd_sweep_x64 and k_tvd_sweep_yz64 below.
 template <class real>
 __global__ __launch_bounds__(256, 1) void k_tvd_sweep_m(const BoxDesc* __restrict__ boxes, Plan plan,
                                                                               TvdSweepArgs<real> a) {
