@@ -299,6 +299,10 @@ int build_plan(imhd_ctx* c, PlanDev& p, int which, int dir, int seg = 0, bool tr
                     lo = normal ? 0 : -1; hi = normal ? n : n + 2; break;
                 case 13:  // passive final update (offset 2)
                     lo = 1; hi = n; break;
+                case 25:  // union of the three predictor flux ranges (k_flux3)
+                    lo = 1 - nb; hi = n + nb; break;
+                case 26:  // union of the three corrector flux ranges (their transverse range)
+                    lo = 3 - nb; hi = n + nb - 2; break;
                 // K98 TVD integrator (isotvd_mod.f90); offset 0 predictor, 2 corrector
                 case 16:  // predictor Roe average / HLLE faces: pencil cells [1-nb, n+nb]
                     lo = 1 - nb; hi = normal ? n + nb - 1 : n + nb; break;
@@ -325,6 +329,8 @@ int build_plan(imhd_ctx* c, PlanDev& p, int which, int dir, int seg = 0, bool tr
                 case 29:  // CT half step and final update: the whole padded box
                 case 30:
                     lo = 1 - nb; hi = n + nb; break;
+                case 14: break;   // below
+                default: FAIL(c, IMHD_EINVAL, "no plan %d", which);
             }
             if (trim) switch (which) {
                 // the interior's final update takes corrector fluxes and corners 0 .. n, they
