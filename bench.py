@@ -322,14 +322,15 @@ FAMILY_SYMBOL = {"flux_pred": "k_flux3", "flux_corr": "k_flux3", "corner_pred": 
                  "pass_stage_corr": "k_pass_stage_z", "fill_ghosts": "k_fill_ghost_band", "ou_forcing": "k_ou_kick"}
 
 
-def kernel_symbol(family, esz, recon="plm"):
+def kernel_symbol(family, esz, recon="plm", riemann="hlld"):
     """The kernel that launches of a family run, None for a family that is not counted.  The
     fused VL stages: the characteristic PPM corrector has its own kernel; the predictor and
-    the PLM corrector have one in FP64; the others run k_vl_stage."""
+    the PLM corrector (but not with the Roe solver) have one in FP64; the others run
+    k_vl_stage."""
     if family in ("stage_pred", "stage_corr", "stage_corr_cfl"):
         if family != "stage_pred" and recon == "ppm_char":
             return "k_vl_char"
-        if esz == 8 and (family == "stage_pred" or recon == "plm"):
+        if esz == 8 and (family == "stage_pred" or (recon == "plm" and riemann != "roe")):
             return "k_vl_near"
         return "k_vl_stage"
     return FAMILY_SYMBOL.get(family)

@@ -72,7 +72,8 @@ __device__ __forceinline__ real stage_face_own(const SweepArgs<real>& a, const r
     }
 }
 // z face k+1/2: predictor between the thread's own cells of planes k (UL) and k+1 (UR),
-// both in registers; correctors load their stencils (holding them spills at 128 VGPRs).
+// both in registers; FP64 PLM corrector with those two of its four stencil cells from
+// registers; the other correctors load their stencils (holding them spills at 128 VGPRs).
 template <class real, int RS, int KIND>
 __device__ __forceinline__ real stage_face_z(const SweepArgs<real>& a, const real* UL, const real* UR, long long c,
                                              long long s, real* F) {
@@ -91,6 +92,13 @@ __device__ __forceinline__ real stage_face_z(const SweepArgs<real>& a, const rea
         return smax;
     } else if constexpr (KIND >= 2) {
         return ppm_flux_calc<real, RS, false>(a, c, s, F);
+    } else if constexpr (sizeof(real) == 8) {
+        real W[4][6];
+        prim_load(a, c - s, W[0]);
+        prim_rot(UL[0], UL[perm(2, 1)], UL[perm(2, 2)], UL[perm(2, 3)], UL[perm(2, 5)], UL[perm(2, 6)], W[1]);
+        prim_rot(UR[0], UR[perm(2, 1)], UR[perm(2, 2)], UR[perm(2, 3)], UR[perm(2, 5)], UR[perm(2, 6)], W[2]);
+        prim_load(a, c + 2 * s, W[3]);
+        return plm_flux<real, RS>(a, W, bn_at(a, c), F);
     } else {
         return flux_corr_calc<real, RS>(a, c, s, F);
     }
@@ -852,7 +860,14 @@ __global__ __launch_bounds__(TX * TY, VS_WAVES) void k_vl_stage(const BoxDesc* _
     if (!PRED && a.cmax != nullptr) atomic_max_nonneg(a.cmax, b, (double)cfl);
 }
 
-// kind: 0 predictor, 1 PLM corrector (both FP32; FP64 runs k_vl_near), 2 PPM-primitive
+// FP64 stages whose faces read near neighbours: k_vl_near, but not the PLM corrector with the
+// Roe solver.  Roe's eigenvectors beside the march's registers spill 151 of 256 there: 720 us
+// per launch at 128^3 (1344 at 190 x 161 x 147) against 571 (1027) in k_vl_stage, which forms its
+// faces one by one and spills none.  HLLD 501 (920) against 589 (1015).
+template <int RS, bool PRED>
+constexpr bool vs_near() { return PRED || RS != RS_ROE; }
+
+// kind: 0 predictor, 1 PLM corrector (FP64: k_vl_near where vs_near), 2 PPM-primitive
 // corrector; the PPM-characteristic corrector runs k_vl_char; shape 2 exists in FP32 only
 template <class real, int RS, int KIND>
 void launch_vl_stage_k(hipStream_t st, const BoxDesc* boxes, const TilePlan& plan, const StageArgs<real>& a,
@@ -895,7 +910,9 @@ int vl_stage_blocks_per_cu(int kind, int shape) {
     if constexpr (sizeof(real) == 8) {
         switch (kind) {
             case 0: return vl_near_blocks_per_cu<RS, true>(shape);
-            case 1: return vl_near_blocks_per_cu<RS, false>(shape);
+            case 1:
+                if constexpr (vs_near<RS, false>()) return vl_near_blocks_per_cu<RS, false>(shape);
+                else return vl_stage_blocks_per_cu_k<real, RS, 1>(shape);
             case 2: return vl_stage_blocks_per_cu_k<real, RS, 2>(shape);
             default: return vl_char_blocks_per_cu<real, RS>(shape);
         }
@@ -918,7 +935,10 @@ void launch_vl_stage(hipStream_t st, const BoxDesc* boxes, const TilePlan& plan,
     if constexpr (sizeof(real) == 8) {
         switch (kind) {
             case 0: launch_vl_near<RS, true>(st, boxes, plan, a, shape); break;
-            case 1: launch_vl_near<RS, false>(st, boxes, plan, a, shape); break;
+            case 1:
+                if constexpr (vs_near<RS, false>()) launch_vl_near<RS, false>(st, boxes, plan, a, shape);
+                else launch_vl_stage_k<real, RS, 1>(st, boxes, plan, a, shape);
+                break;
             case 2: launch_vl_stage_k<real, RS, 2>(st, boxes, plan, a, shape); break;
             default: launch_vl_char<real, RS>(st, boxes, plan, a, shape); break;
         }

@@ -27,6 +27,11 @@ def test_symbol_is_the_launched_kernel(family, esz, recon, kernel):
     assert any(re.search(r"__global__[^;{]*\b" + kernel + r"\(", t) for t in sources().values())
 
 
+def test_roe_plm_corrector_in_fp64():
+    assert bench.kernel_symbol("stage_corr", 8, "plm", "roe") == "k_vl_stage"
+    assert bench.kernel_symbol("stage_pred", 8, "plm", "roe") == "k_vl_near"
+
+
 def test_families_are_profiled_by_the_library():
     api = sources()["imhd_api.cpp"]
     for family in list(bench.FAMILY_SYMBOL) + ["stage_pred", "stage_corr", "stage_corr_cfl"]:
