@@ -11,9 +11,16 @@ namespace imhd {
 // then y, then z over whole planes; the composition equals reading every ghost cell
 // from (map_x(i), map_y(j), map_z(k)) with an independent per-axis source map, which is
 // what this kernel does in one pass (sources are always interior cells).
+// FEW: a periodic box of fewer cells than ghost layers, where the reference's source can be a
+// ghost cell, which it has filled before: the interior cell that this one holds is more than
+// one box length away.  (Divisions, 1 us at 190 x 161 x 147, so not for the other boxes.)
+template <bool FEW>
 __device__ __forceinline__ int bc_map(int i, int n, int bc) {
     if (i >= 1 && i <= n) return i;
-    if (bc == 2) return i < 1 ? i + n : i - n;   // periodic: q(-g) = q(n-g), q(n+1+g) = q(1+g)
+    if (bc == 2) {   // periodic: q(-g) = q(n-g), q(n+1+g) = q(1+g)
+        if (FEW) return i < 1 ? n - (-i) % n : (i - 1) % n + 1;
+        return i < 1 ? i + n : i - n;
+    }
     return i < 1 ? 1 : n;                         // open: copy the edge cell
 }
 
@@ -69,29 +76,31 @@ __device__ __forceinline__ void band_cell(const BoxDesc& B, unsigned t, int w, i
 __device__ __forceinline__ bool within(const BoxDesc& B, int i, int j, int k, int w) {
     return i >= 1 - w && j >= 1 - w && k >= 1 - w && i <= B.n[0] + w && j <= B.n[1] + w && k <= B.n[2] + w;
 }
+template <bool FEW>
 __device__ __forceinline__ long long ghost_source(const BoxDesc& B, int i, int j, int k) {
-    return cell_index(B, bc_map(i, B.n[0], B.bc), bc_map(j, B.n[1], B.bc), bc_map(k, B.n[2], B.bc));
+    return cell_index(B, bc_map<FEW>(i, B.n[0], B.bc), bc_map<FEW>(j, B.n[1], B.bc), bc_map<FEW>(k, B.n[2], B.bc));
 }
 
 // The plan gives each box r[0] = number of cells of its band of depth a.depth
-template <class real>
+template <class real, bool FEW>
 __global__ __launch_bounds__(256) void k_fill_ghost_band(const BoxDesc* __restrict__ boxes, Plan plan, GhostArgs<real> a) {
     int b, g, dum1, dum2, i, j, k;
     if (!plan_item(plan, b, g, dum1, dum2)) return;
     const BoxDesc& B = boxes[b];
     band_cell(B, (unsigned)g, a.depth, i, j, k);
-    const long long d = cell_index(B, i, j, k), s = ghost_source(B, i, j, k);
+    const long long d = cell_index(B, i, j, k), s = ghost_source<FEW>(B, i, j, k);
     copy_fields(a, within(B, i, j, k, a.depth2) ? a.nreal2 : a.nreal, d, s);
 }
 
-// The same for the compensation terms of the FP32 state, to depth a.depth2 only (same plan)
+// The same for the compensation terms of the FP32 state, to depth a.depth2 only (same plan); no
+// box has fewer cells than ghost layers
 __global__ __launch_bounds__(256) void k_fill_comp_ghosts(const BoxDesc* __restrict__ boxes, Plan plan, CompGhostArgs a) {
     int b, g, dum1, dum2, i, j, k;
     if (!plan_item(plan, b, g, dum1, dum2)) return;
     const BoxDesc& B = boxes[b];
     band_cell(B, (unsigned)g, a.depth, i, j, k);
     if (!within(B, i, j, k, a.depth2)) return;
-    const long long d = cell_index(B, i, j, k), s = ghost_source(B, i, j, k);
+    const long long d = cell_index(B, i, j, k), s = ghost_source<false>(B, i, j, k);
     float v[4];
 #pragma unroll
     for (int f = 0; f < 4; f++) v[f] = a.comp[f][s];
@@ -644,7 +653,9 @@ template void launch_prot_fix<float>(const Launch&, const ProtArgs<float>&);
 
 template <class real>
 void launch_fill_ghost_band(const Launch& L, const GhostArgs<real>& a) {
-    if (L.plan.total > 0) L256((k_fill_ghost_band<real>), L.boxes, L.plan, a);
+    if (L.plan.total <= 0) return;
+    if (a.few) L256((k_fill_ghost_band<real, true>), L.boxes, L.plan, a);
+    else L256((k_fill_ghost_band<real, false>), L.boxes, L.plan, a);
 }
 void launch_fill_comp_ghosts(const Launch& L, const CompGhostArgs& a) {
     if (L.plan.total > 0) L256(k_fill_comp_ghosts, L.boxes, L.plan, a);

@@ -19,6 +19,7 @@ struct GhostArgs {
     double* d[3];
     int nreal, depth;     // fields r[0 .. nreal) and d, to this depth
     int nreal2, depth2;   // and r[nreal .. nreal2), the passives, to depth2 <= depth
+    bool few;             // a box has fewer cells than depth along an axis
 };
 
 struct CompGhostArgs {

@@ -1052,6 +1052,7 @@ void fill_ghosts(imhd_ctx* c) {
     g.depth = c->hb[0].nb;
     g.nreal2 = 7 + c->cfg.npass;
     g.depth2 = 3;   // passive_mod.f90:52
+    for (const BoxDesc& B : c->hb) g.few = g.few || std::min(B.n[0], std::min(B.n[1], B.n[2])) < B.nb;
     launch_fill_ghost_band<real>(mk(c, c->pl_gband), g);
 }
 
