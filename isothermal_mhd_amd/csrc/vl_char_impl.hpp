@@ -27,17 +27,18 @@
 // are formed where they are used: hoisted out of the march they took 70 registers.  FP64 reads
 // the own column's planes k, k+2 and k+3 again from L2 each plane for the same reason; FP32 has
 // the registers to carry them and loads plane k+3 only, at the start of the pass.
-// FP64: two workgroups per CU (75 KB of LDS per 16 x 16 tile, 256 registers): the 65 registers
-// that spill cost less than the second workgroup gains (128^3: 1.10 ms per launch, against
-// 1.36 ms with one workgroup and nothing spilled).
+// FP64: two workgroups per CU (75 KB of LDS per 16 x 16 tile, 256 registers): the 63 registers
+// that spill cost less than the second workgroup gains (128^3, full ranges in four rounds of
+// segments: 1.10 ms per launch, against 1.36 ms with one workgroup and nothing spilled).
 //
-// Measured per launch at 128^3 (HLLD), against the per-face form: 2.02 -> 1.10 ms.
+// Measured per launch at 128^3 (HLLD), against the per-face form: 2.02 -> 1.10 ms, 0.95 over the
+// ranges of a native step in one round of segments; the VALU is busy in 57 % of the cycles.
 //
 // FP32 is the same kernel with the fused operations of the per-face form written out
 // (char_edge, ppm_edge, char_solve), so that its results keep their bits: a rounding moved in
 // an edge value turns up as a different limiter branch in single cells.  Per launch at 256^3
-// (HLLD) 4.02 -> 2.76 ms with 16 x 16 tiles, 2.61 with the own column carried.  It is bound by
-// VALU issue (5470 instructions per cell before the carry, the VALU busy in 90 % of the cycles);
+// (HLLD) 4.02 -> 2.76 ms with 16 x 16 tiles, 2.60 with the own column carried.  It is bound by
+// VALU issue (5206 instructions per cell, the VALU busy in 90 % of the cycles);
 // four waves per SIMD, by lane shifts in place of 8 KB of LDS, spill 99 registers: 3.5 ms.
 #pragma once
 #include "vl_stage_impl.hpp"
@@ -273,10 +274,8 @@ __device__ __forceinline__ double lane_next_r(double x) { return lane_next_d(x);
 __device__ __forceinline__ float lane_prev_r(float x) { return lane_prev(x); }
 __device__ __forceinline__ float lane_next_r(float x) { return lane_next(x); }
 
-// Waves per SIMD.  FP64: 75 KB of LDS per 16 x 16 tile and 256 registers give two workgroups
-// per CU; the 65 registers that spill cost less than the second workgroup gains (128^3:
-// 1.10 ms per launch against 1.36 ms with one workgroup and none spilled).  FP32: 45 KB per
-// 16 x 16 tile and 168 registers, three workgroups; 32 x 16 (88 KB) fits one, at two.
+// Waves per SIMD (above).  FP64: two, 75 KB of LDS per 16 x 16 tile and 256 registers.  FP32: 45
+// KB per 16 x 16 tile and 168 registers, three; 32 x 16 (88 KB) fits one workgroup, at two.
 template <class real, int N>
 constexpr int vc_waves() { return sizeof(real) == 4 && N == 256 ? 3 : 2; }
 

@@ -16,8 +16,9 @@
 //     states, and what else only x-neighbours read, come by lane shift; a plane's upper z-state
 //     is carried to the next plane's face;
 //   - everything of plane k+2 is loaded at the start of the pass that solves plane k+1.
-// HLLD at 190 x 161 x 147, against the per-face form (k_vl_stage): predictor 0.72 -> 0.655 ms,
-// corrector 0.98 -> 0.945.
+// HLLD at 190 x 161 x 147, against the per-face form (k_vl_stage) over the same ranges: predictor
+// 0.72 -> 0.655 ms, corrector 0.98 -> 0.945; in one round of segments 0.61 and 0.89.  The VALU is
+// busy in 60 % of the cycles.  Not for the PLM corrector with the Roe solver (vs_near).
 // Per plane k of the march:
 //   A  the y- and x-faces of plane k+1 and the z-face k+1/2
 //   D  corner EMFs of index k; plane k+2 replaces plane k+1 in LDS, its centre values are formed
