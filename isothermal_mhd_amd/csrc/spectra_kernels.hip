@@ -107,8 +107,9 @@ __global__ __launch_bounds__(256) void k_spec_bin(const float* __restrict__ s, i
 // HIST_LDS_BINS) the other lanes then add for themselves, which the LDS serialises only
 // among equal bins (a ballot per distinct bin of the wave, up to 64 in turn, made a broad
 // distribution 149 us at 256^3 FP32, 63 so; few populated bins are no slower either: a call
-// with 2 to 4 takes 85 to 89 us, 101 to 111 with a ballot each); straight into the global counts, for more bins,
-// every distinct bin has its ballot.  Counts are exact integers, so the order does not matter.
+// with 2 to 4 takes 85 to 89 us, 101 to 111 with a ballot each); straight into the global
+// counts, for more bins, every distinct bin has its ballot.  Counts are exact integers, so the
+// order does not matter.
 constexpr int HIST_LDS_BINS = 4096;
 template <class real, bool LDS>
 __global__ __launch_bounds__(256) void k_density_hist(BoxDesc B, const real* __restrict__ rho, float drho, int nbins,
